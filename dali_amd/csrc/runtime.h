@@ -50,6 +50,20 @@ int sgemm_dma_stream(bool ta, bool tb, int M, int N, int nseg, const int* K, con
 // sgemm_dma128.hip: row-major C[M, N] = alpha * A . B + beta * C over whole 32-deep slabs with 128x128 tiles, one workgroup per
 // compute unit walking a list of tiles (ta: A stored as [K][M]; tb: B stored as [N][K]). Same return values.
 int sgemm_dma128(bool ta, bool tb, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float alpha, float beta, float* C, int ldc, int cus);
+// Output row map (convolution over a padded image computed at every padded position): row m stands for position (n, i, j) of an
+// [., hw / w, w] grid; only i < oh, j < ow are stored, at row (n * oh + i) * ow + j. hw and w come with the multiplier / shift of
+// an exact division (sgemm_row_map_div).
+struct SgemmRowMap {
+    int on;
+    unsigned hw, hw_m, w, w_m;
+    int hw_s, w_s, oh, ow;
+};
+// n / d for n < 2^31: m = ceil(2^(31+s) / d) with 2^(s-1) < d <= 2^s, computed by the launcher
+__device__ __forceinline__ unsigned sgemm_row_map_div(unsigned n, unsigned m, int s) { return (unsigned)(((unsigned long long)n * m) >> (31 + s)); }
+// sgemm_split.hip: row-major C[M, N] = alpha * sum_s A_s . B_s + beta * C on the bf16 matrix cores, every fp32 value cut into three
+// bf16 pieces that add up to it. Same return values.
+int sgemm_split(bool ta, bool tb, int M, int N, int nseg, const int* K, const float* const* A, const int* lda, const float* const* B, const int* ldb, float alpha,
+                float beta, float* C, int ldc, const SgemmRowMap& map, int cus);
 // hipFuncSetAttribute(MaxDynamicSharedMemorySize) once per kernel: later launches of that kernel, which may be recorded into a
 // graph, are launches only. Keyed on the kernel's address (kernels of one signature share a function type, so a flag inside a
 // generic lambda or template would be shared among them).

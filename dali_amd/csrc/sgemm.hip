@@ -82,16 +82,8 @@ struct GemmArgs {
     float* c_out;
     float* h_out;
     int H;
-    // Output row map (convolution over a padded image computed at every padded position): row m stands for position
-    // (n, i, j) of an [., map_h, map_w] grid; only i < map_oh, j < map_ow are stored, at row (n * map_oh + i) * map_ow + j.
-    // hw = map_h * map_w and map_w come with the multiplier / shift of an exact division (see row_map_div).
-    int map_on;
-    unsigned map_hw, map_hw_m, map_w, map_w_m;
-    int map_hw_s, map_w_s, map_oh, map_ow;
+    SgemmRowMap map;  // only the multi-term kernels carry it
 };
-
-// n / d for n < 2^31: m = ceil(2^(31+s) / d) with 2^(s-1) < d <= 2^s, computed by the launcher
-__device__ __forceinline__ unsigned row_map_div(unsigned n, unsigned m, int s) { return (unsigned)(((unsigned long long)n * m) >> (31 + s)); }
 
 __device__ __forceinline__ void publish(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float observe(const float* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -726,11 +718,11 @@ __global__ __launch_bounds__(256 * KW, (BM == 128 && !EDGE && KW == 1) ? 2 : 1) 
                 int m = m0 + wm * WTM + ii * 32 + 8 * (v / 4) + 4 * h + (v % 4);
                 if (m < M) {
                     size_t out_row = (size_t)m;
-                    if (MAXSEG > 2 && g.map_on) {  // only the multi-term kernels carry the map
-                        const unsigned img = row_map_div((unsigned)m, g.map_hw_m, g.map_hw_s), rest = (unsigned)m - img * g.map_hw;
-                        const unsigned i = row_map_div(rest, g.map_w_m, g.map_w_s), j = rest - i * g.map_w;
-                        if ((int)i >= g.map_oh || (int)j >= g.map_ow) continue;
-                        out_row = ((size_t)img * g.map_oh + i) * g.map_ow + j;
+                    if (MAXSEG > 2 && g.map.on) {  // only the multi-term kernels carry the map
+                        const unsigned img = sgemm_row_map_div((unsigned)m, g.map.hw_m, g.map.hw_s), rest = (unsigned)m - img * g.map.hw;
+                        const unsigned i = sgemm_row_map_div(rest, g.map.w_m, g.map.w_s), j = rest - i * g.map.w;
+                        if ((int)i >= g.map.oh || (int)j >= g.map.ow) continue;
+                        out_row = ((size_t)img * g.map.oh + i) * g.map.ow + j;
                     }
                     float* c = g.C + out_row * g.ldc + n;
                     const float sum = acc[0][ii][jj][v];  // (with split-K: the fold above)
@@ -774,7 +766,7 @@ static int launch_tile(GemmArgs g, bool ta, bool tb, bool vec, int split_k, bool
         else if (V_)                                                                                        \
             hipLaunchKernelGGL((sgemm_kernel<BM, BN, BK, false, TB_, true, DEPTH, false, KW, MIDB, false, kMaxSeg>), grid, block, pad_lds, st, g); \
     }
-    if (g.nseg > 2 || g.map_on) {
+    if (g.nseg > 2 || g.map.on) {
         if (ta) return fail("sgemm: more than two terms, or an output row map, need a left operand stored by rows");
         DALI_GEMM_CASE_TERMS(false, true)
         DALI_GEMM_CASE_TERMS(false, false)
@@ -814,8 +806,8 @@ static int run_tile(const GemmArgs& g, bool ta, bool tb, bool vec, int split_k) 
         same_ld = same_ld && g.seg[s].lda == g.seg[0].lda && g.seg[s].ldb == g.seg[0].ldb;
     }
     constexpr bool dma_tile = BM == 64 && BN == 64 && BK == 64 && KW == 2 && !MIDB;
-    if (!fast || (!same_ld && !(dma_tile && split_k == 1 && g.nseg <= 2 && !g.map_on))) return launch_tile<BM, BN, BK, DEPTH, KW, MIDB>(g, ta, tb, vec, split_k, true);
-    if (dma_tile && split_k == 1 && g.nseg <= 2 && !g.map_on) {
+    if (!fast || (!same_ld && !(dma_tile && split_k == 1 && g.nseg <= 2 && !g.map.on))) return launch_tile<BM, BN, BK, DEPTH, KW, MIDB>(g, ta, tb, vec, split_k, true);
+    if (dma_tile && split_k == 1 && g.nseg <= 2 && !g.map.on) {
         // inner extents that end in a partly filled slab: the same kernel fills what is missing with zeros as the slab arrives,
         // instead of a second launch for the rest ([256,1000].[1000,4000] twice: 47.7 -> 38 us)
         bool partly = false;
@@ -851,7 +843,7 @@ static int run_tile(const GemmArgs& g, bool ta, bool tb, bool vec, int split_k) 
     if (whole.nseg > 0) {
         int st = 0;
         bool done = false;
-        if (dma_tile && split_k == 1 && whole.nseg <= 2 && !whole.map_on) {
+        if (dma_tile && split_k == 1 && whole.nseg <= 2 && !whole.map.on) {
             // small grids of whole slabs: the kernel that has its operand slabs written into LDS by the loads themselves
             const float* as[2] = {whole.seg[0].A, whole.seg[1].A};
             const float* bs[2] = {whole.seg[0].B, whole.seg[1].B};
@@ -1015,19 +1007,35 @@ static int sgemm_rowmajor(int nseg, bool ta, bool tb, int M, int N, const int* K
             *m = (unsigned)((((unsigned long long)1 << (31 + sft)) + d - 1) / d);
             *sh = sft;
         };
-        g.map_on = 1;
-        g.map_hw = (unsigned)(map_h * map_w);
-        g.map_w = (unsigned)map_w;
-        set_div(g.map_hw, &g.map_hw_m, &g.map_hw_s);
-        set_div(g.map_w, &g.map_w_m, &g.map_w_s);
-        g.map_oh = row_map[2];
-        g.map_ow = row_map[3];
+        g.map.on = 1;
+        g.map.hw = (unsigned)(map_h * map_w);
+        g.map.w = (unsigned)map_w;
+        set_div(g.map.hw, &g.map.hw_m, &g.map.hw_s);
+        set_div(g.map.w, &g.map.w_m, &g.map.w_s);
+        g.map.oh = row_map[2];
+        g.map.ow = row_map[3];
     }
     if (g.nseg == 0) {
         // empty inner extent: C = beta * C
         g.nseg = 1;
         g.seg[0].K = 0;
         vec = false;
+    }
+    if (g.seg[0].K > 0) {
+        // large products through the bf16 matrix cores: six products of the pieces of values cut in three take less time there than
+        // the one product on the fp32 ones ([256,32000] over K = 1024: 105 against 159 us; the sizes are judged there)
+        const float* as[kMaxSeg];
+        const float* bs[kMaxSeg];
+        int ks[kMaxSeg], las[kMaxSeg], lbs[kMaxSeg];
+        for (int s = 0; s < g.nseg; ++s) {
+            as[s] = g.seg[s].A;
+            bs[s] = g.seg[s].B;
+            ks[s] = g.seg[s].K;
+            las[s] = g.seg[s].lda;
+            lbs[s] = g.seg[s].ldb;
+        }
+        const int r = sgemm_split(ta, tb, M, N, g.nseg, ks, as, las, bs, lbs, alpha, beta, C, ldc, g.map, device_cus());
+        if (r != 0) return r > 0 ? DALI_HIP_OK : DALI_HIP_ERROR;
     }
     // More than `low_rows_from` and at most 64 rows against a wide B stored [K][N]: bound by the matrix pipe rather than by
     // streaming B, so 64-row tiles fed through LDS, one workgroup per compute unit ([64,1024].[1024,32000]: 45 -> 41 us, 0.65 of the fp32 matrix peak; the row-streaming
@@ -1095,7 +1103,7 @@ static int sgemm_rowmajor(int nseg, bool ta, bool tb, int M, int N, const int* K
     static const int variant = getenv("DALI_HIP_GEMM_VARIANT") ? atoi(getenv("DALI_HIP_GEMM_VARIANT")) : 0;
     // >0: that many shares of the inner extent through the streaming kernel for every product it takes; <0: never
     static const int stream_env = getenv("DALI_HIP_GEMM_STREAM") ? atoi(getenv("DALI_HIP_GEMM_STREAM")) : 0;
-    const bool stream_fits = vec && g.nseg <= 2 && !g.map_on && !rows_may_overlap;
+    const bool stream_fits = vec && g.nseg <= 2 && !g.map.on && !rows_may_overlap;
     if (stream_env > 0 && stream_fits) {
         const int st = stream_product(g, ta, tb, stream_env);
         if (st >= 0) return st;
@@ -1108,7 +1116,7 @@ static int sgemm_rowmajor(int nseg, bool ta, bool tb, int M, int N, const int* K
     const long rounds64 = (tiles64_all + cus_all - 1) / cus_all;
     const bool uneven64 = tiles128 >= 64 && g.nseg == 1 && g.seg[0].K >= 2048 && (double)tiles64_all < 0.8 * (double)(rounds64 * cus_all);
     if (tiles128 >= 192 || uneven64) {
-        if (vec && g.nseg == 1 && !g.map_on && !rows_may_overlap) {
+        if (vec && g.nseg == 1 && !g.map.on && !rows_may_overlap) {
             const int st = tiles128_product(g, ta, tb);
             if (st >= 0) return st;
         }

@@ -1,0 +1,509 @@
+// fp32 GEMM on the bf16 matrix cores: every operand value is cut into three bf16 pieces whose sum is the value itself.
+//
+// Row-major view: C[M,N] = alpha * sum_s A_s[M,K_s] * B_s[K_s,N] + beta * C with A stored [M][K] or [K][M] and B stored [K][N] or [N][K].
+//
+// What bounds the kernels it stands in for is the fp32 matrix rate (157 TFLOP/s; a bf16 instruction does sixteen times as much per
+// cycle). With h = bf16(x), m = bf16(x - h), l = x - h - m, all rounded to nearest, x = h + m + l holds exactly: 24 significant
+// bits in three times 8, and the exponent range of bf16 is that of fp32. Of the nine products of the pieces of a and b the six
+// of weight 2^-16 and more are summed (hh, hm, mh, hl, lh, mm); those left out, ml + lm + ll, come to at most 2^-26 |a b|, a quarter of
+// what rounding one fp32 product may cost. Products of bf16 pieces are exact in fp32 and the sums are kept in fp32.
+//
+// Where the pieces do not represent the value the tile is redone with the fp32 instructions (`redo`): infinities, NaN and values that
+// round to infinity in bf16 leave a sum that is not finite; values whose last piece falls below the smallest bf16 leave
+// bits in the low half of that piece, which the cutting collects. So are tiles whose sums overflow.
+//
+// What a MFMA of this kind adds to its accumulator is rounded more coarsely than a chain of fp32 instructions would: over a whole
+// inner extent of 512 the sums were 3.4e-7 from double precision against 1.5e-7 for the fp32 kernels. So a chain covers two slabs only
+// (32 values of k, smallest products first) and is then added to the sums by the vector unit: 1.07e-7 (normal values, K = 512;
+// K = 133: 0.83e-7 against 1.11e-7, K = 1999: 1.2e-7 against 2.1e-7, K = 32000: 2.9e-7 against 5.7e-7).
+//
+// A workgroup of four waves owns a 128x128 tile, a wave 64x64 of it as 2x2 accumulators of v_mfma_f32_32x32x16_bf16. Slabs of 16
+// values of k come through registers (fetched two slabs ahead), are cut there, once per workgroup and value, and written to
+// LDS as three planes of [row][16 k] in bf16: whatever the storage order, a lane packs neighbours in k, so the transposition of
+// [K][x] operands costs nothing. Two stages of 24 KiB, one barrier per slab: while a slab is multiplied the next one is cut. 48 KiB
+// and at most 256 registers: two workgroups share a compute unit.
+//
+// Measured (random operands): [256,1024].[1024,32000] 159 -> 105 us, its gradients [1024,256].[256,32000] 149 -> 123 us and
+// [256,32000].[32000,1024] 146 -> 104 us; 4096^3 with B stored [N][K] 950 -> 740 us (186 TFLOP/s), [K][N] 970 -> 884 us. The matrix instructions alone take
+// 490 us of that (the card holds about 1.75 GHz under them); cutting and writing to LDS is what does not hide behind them: with one
+// of the six products 390 us, without cutting 640. Measured and dropped: separate sums for the small products (no more accurate and
+// no faster), slabs of 32 with two barriers, three stages with operands read ahead of the barrier (790 us), subtracting with
+// v_dot2_f32_bf16 (slower and not exact).
+//
+// LDS rows are 32 bytes, two 16-byte granules of eight k. Granule g of row r lies in slot g ^ (bit 2 of r) of the row whose bit 2 is
+// flipped where bit 3 of r is set: eight neighbouring rows touch eight different 16-byte columns of 128 bytes, sixteen touch sixteen of
+// 256, when reading and when writing.
+#include <cstdlib>
+#include <type_traits>
+
+#include "runtime.h"
+
+namespace dali_hip {
+namespace {
+
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int uintx4 __attribute__((ext_vector_type(4)));
+// loads claim element alignment only: any leading dimension, any view
+typedef floatx4 floatx4u __attribute__((aligned(4)));
+
+constexpr int kTile = 128, kSlab = 16;
+constexpr int kRowBytes = kSlab * 2;
+constexpr int kPlaneBytes = kTile * kSlab * 2;     // one piece of one operand
+constexpr int kOperandBytes = 3 * kPlaneBytes;
+constexpr int kStageBytes = 2 * kOperandBytes;     // the pieces of one slab of both operands; two stages
+constexpr int kMaxTerms = 8;
+
+struct SplitArgs {
+    const float* A[kMaxTerms];
+    const float* B[kMaxTerms];
+    int lda[kMaxTerms], ldb[kMaxTerms], K[kMaxTerms];
+    int nseg;
+    int M, N;
+    float* C;
+    int ldc;
+    float alpha, beta;
+    int tiles_m, tiles_n, shares;
+    int slabs;        // of all terms together
+    float* partials;  // shares > 1: [share][tile][16384], else unused
+    SgemmRowMap map;
+};
+
+__device__ __forceinline__ float lo_part(unsigned int pair) { return __uint_as_float(pair << 16); }
+__device__ __forceinline__ float hi_part(unsigned int pair) { return __uint_as_float(pair & 0xffff0000u); }
+__device__ __forceinline__ unsigned int pack2(float a, float b) {
+    const floatx2 v = {a, b};
+    return __builtin_bit_cast(unsigned int, __builtin_convertvector(v, bf16x2));
+}
+
+// two neighbours in k cut into their three pieces; `lost` collects what the last piece cannot hold (its low half)
+__device__ __forceinline__ void cut2(float a, float b, unsigned int& h, unsigned int& m, unsigned int& l, unsigned int& lost) {
+    h = pack2(a, b);
+    const float a1 = a - lo_part(h), b1 = b - hi_part(h);
+    m = pack2(a1, b1);
+    const float a2 = a1 - lo_part(m), b2 = b1 - hi_part(m);
+    l = pack2(a2, b2);
+    lost |= __float_as_uint(a2) | __float_as_uint(b2);
+}
+
+__device__ __forceinline__ int lds_offset(int row, int granule) {
+    return (row ^ (((row >> 3) & 1) << 2)) * kRowBytes + ((granule ^ ((row >> 2) & 1)) << 4);
+}
+
+// A thread's share of one operand's slab: eight k of one row (column) of the tile, one granule of each plane.
+//   KROWS (stored [x][K]): row t / 2, k from 8 (t % 2): two 16-byte loads
+//   else  (stored [K][x]): column t % 128, k from 8 (t / 128): eight loads of neighbouring columns
+template <bool KROWS>
+struct Loader {
+    int row, granule;  // within the tile
+    unsigned off;      // of the first value, from the operand's first row and the slab's first k (KROWS), or from the slab's first k
+
+    __device__ __forceinline__ void init(int tid, int x0, int x_end, int ld) {
+        row = KROWS ? tid >> 1 : tid & 127;
+        granule = KROWS ? tid & 1 : tid >> 7;
+        set_ld(x0, x_end, ld);
+    }
+    // (rows past the end repeat the last one; what they sum up to is not stored)
+    __device__ __forceinline__ void set_ld(int x0, int x_end, int ld) {
+        const int x = min(x0 + row, x_end - 1);
+        off = KROWS ? (unsigned)((x - x0) * ld + 8 * granule) : (unsigned)(8 * granule * ld + x);
+    }
+    // `p`: the tile's first row at the slab's first k (KROWS), the slab's first k (else)
+    __device__ __forceinline__ void fetch(float* v, const float* p, int ld) const {
+        if (KROWS) {
+            const floatx4 a = *(const floatx4u*)(p + off), b = *(const floatx4u*)(p + off + 4);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[j] = a[j];
+                v[4 + j] = b[j];
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = (p + (size_t)j * ld)[off];  // (the row in scalar registers)
+        }
+    }
+    // the last, partly filled slab of a term: `left` values of k, the others are zero
+    __device__ __forceinline__ void fetch_tail(float* v, const float* p, int ld, int left) const {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int k = 8 * granule + j, back = max(k - (left - 1), 0);
+            const float a = p[off + (unsigned)(KROWS ? j : j * ld) - (unsigned)(KROWS ? back : back * ld)];
+            v[j] = k < left ? a : 0.0f;
+        }
+    }
+    __device__ __forceinline__ void store_cut(const float* v, char* lds, unsigned int& lost) const {
+        uintx4 h, m, l;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            unsigned int hq, mq, lq;
+            cut2(v[2 * q], v[2 * q + 1], hq, mq, lq, lost);
+            h[q] = hq;
+            m[q] = mq;
+            l[q] = lq;
+        }
+        char* d = lds + lds_offset(row, granule);
+        *(uintx4*)d = h;
+        *(uintx4*)(d + kPlaneBytes) = m;
+        *(uintx4*)(d + 2 * kPlaneBytes) = l;
+    }
+    // as fp32, rows of 16 k and a pitch of 17 (the redo path)
+    __device__ __forceinline__ void store_plain(const float* v, float* lds) const {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) lds[row * 17 + 8 * granule + j] = v[j];
+    }
+};
+
+// Walks the slabs of the terms in order for the loads, which are the same instructions for every slab, so that the waits for one
+// slab leave the next ones' loads in flight: a partly filled last slab is fetched sixteen values of k ending at the last (what that
+// gets wrong is fetched again when it is cut), and behind the last slab of the share that one is fetched again.
+template <bool TA, bool TB>
+struct Walk {
+    Loader<!TA> a;
+    Loader<TB> b;
+    const float *pa, *pb;
+    int term, left, lda, ldb, todo;  // left: values of k of the term from this slab on; todo: slabs to move on to
+
+    __device__ __forceinline__ void enter(const SplitArgs& g, int k0, int m0, int n0) {
+        lda = g.lda[term];
+        ldb = g.ldb[term];
+        a.set_ld(m0, g.M, lda);
+        b.set_ld(n0, g.N, ldb);
+        left = g.K[term] - k0;
+        k0 = min(k0, g.K[term] - kSlab);
+        pa = g.A[term] + (TA ? (size_t)k0 * lda : (size_t)m0 * lda + k0);
+        pb = g.B[term] + (TB ? (size_t)n0 * ldb + k0 : (size_t)k0 * ldb);
+    }
+    __device__ __forceinline__ void start(const SplitArgs& g, int first_term, int k0, int count, int m0, int n0) {
+        term = first_term;
+        todo = count - 1;
+        enter(g, k0, m0, n0);
+    }
+    // fetches the slab and moves on to the next
+    __device__ __forceinline__ void fetch(const SplitArgs& g, float* va, float* vb, int m0, int n0) {
+        a.fetch(va, pa, lda);
+        b.fetch(vb, pb, ldb);
+        if (todo > 0) {
+            --todo;
+            left -= kSlab;
+            if (left > 0) {
+                const int by = min(left, kSlab);
+                pa += TA ? (size_t)by * lda : (size_t)by;
+                pb += TB ? (size_t)by : (size_t)by * ldb;
+            } else {
+                ++term;
+                enter(g, 0, m0, n0);
+            }
+        }
+    }
+};
+
+// The same walk for the cutting, one to three slabs behind: tells the partly filled slabs.
+template <bool TA, bool TB>
+struct Cutter {
+    int term, left;
+    __device__ __forceinline__ void start(const SplitArgs& g, int first_term, int k0) {
+        term = first_term;
+        left = g.K[term] - k0;
+    }
+    // the slab in `va`, `vb` with zeros behind the end of the term
+    __device__ __forceinline__ void settle(const SplitArgs& g, const Walk<TA, TB>& w, float* va, float* vb, int m0, int n0) {
+        if (left > 0 && left < kSlab) {
+            Loader<!TA> a = w.a;
+            Loader<TB> b = w.b;
+            const int lda = g.lda[term], ldb = g.ldb[term], k0 = g.K[term] - left;
+            a.set_ld(m0, g.M, lda);
+            b.set_ld(n0, g.N, ldb);
+            a.fetch_tail(va, g.A[term] + (TA ? (size_t)k0 * lda : (size_t)m0 * lda + k0), lda, left);
+            b.fetch_tail(vb, g.B[term] + (TB ? (size_t)n0 * ldb + k0 : (size_t)k0 * ldb), ldb, left);
+        }
+        left -= kSlab;
+        if (left <= 0 && term + 1 < g.nseg) left = g.K[++term];
+    }
+};
+
+// LDS written by this wave is there and every wave has come here; loads from global memory stay in flight
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+__device__ __forceinline__ void put(const SplitArgs& g, float* d, float sum) {
+    float r = g.alpha * sum;
+    if (g.beta != 0.0f) r += g.beta * *d;
+    *d = r;
+}
+
+__device__ __forceinline__ void store_result(const SplitArgs& g, int m, int n, float sum) {
+    size_t row = (size_t)m;
+    if (g.map.on) {
+        const unsigned img = sgemm_row_map_div((unsigned)m, g.map.hw_m, g.map.hw_s), rest = (unsigned)m - img * g.map.hw;
+        const unsigned i = sgemm_row_map_div(rest, g.map.w_m, g.map.w_s), j = rest - i * g.map.w;
+        if ((int)i >= g.map.oh || (int)j >= g.map.ow) return;
+        row = ((size_t)img * g.map.oh + i) * g.map.ow + j;
+    }
+    put(g, g.C + row * g.ldc + n, sum);
+}
+
+template <bool TA, bool TB>
+__global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
+    __shared__ __attribute__((aligned(16))) char lds[2 * kStageBytes];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // Every eighth workgroup runs on the same die: a die takes a run of neighbouring tiles (of one share), eight rows of tiles to
+    // a band, and finds the operands its other workgroups asked for in its L2.
+    const int total = g.tiles_m * g.tiles_n * g.shares;
+    int id = blockIdx.x;
+    const int per = total >> 3;
+    if (id < per * 8) id = (id & 7) * per + (id >> 3);
+    const int tiles = g.tiles_m * g.tiles_n;
+    // (the quotients come out of the vector unit)
+    auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+    const int share = uniform(id / tiles);
+    const int tile = id - share * tiles;
+    const int band = uniform(tile / (8 * g.tiles_n)), band_rows = min(8, g.tiles_m - 8 * band), in_band = tile - band * 8 * g.tiles_n;
+    const int tn = uniform(in_band / band_rows), tm = 8 * band + in_band - tn * band_rows;
+    const int m0 = tm * kTile, n0 = tn * kTile;
+    const int s_begin = uniform(g.slabs * share / g.shares), s_end = uniform(g.slabs * (share + 1) / g.shares);
+
+    floatx16 acc[2][2], part[2][2];  // the sums; those of the pair of slabs at hand
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = floatx16{};
+    const int wm = 64 * (wave >> 1), wn = 64 * (wave & 1);
+    unsigned int lost = 0;
+    Walk<TA, TB> w;
+    w.a.init(tid, m0, g.M, 0);
+    w.b.init(tid, n0, g.N, 0);
+    int first_term = 0, first_k = s_begin;
+    while (first_term + 1 < g.nseg && first_k >= (g.K[first_term] + kSlab - 1) / kSlab) first_k -= (g.K[first_term++] + kSlab - 1) / kSlab;
+    first_k *= kSlab;
+    const int count = s_end - s_begin;
+    w.start(g, first_term, first_k, count, m0, n0);
+    Cutter<TA, TB> c;
+    c.start(g, first_term, first_k);
+    float va[2][8], vb[2][8];  // slabs of even and odd number (counted from s_begin)
+    const char* ra = lds + lds_offset(wm + (lane & 31), lane >> 5);
+    const char* rb = lds + kOperandBytes + lds_offset(wn + (lane & 31), lane >> 5);
+
+    // slab `P` (its parity) from LDS through the matrix instructions; meanwhile the next one is cut and written to the other buffer
+    auto multiply = [&](auto parity) {
+        constexpr int P = decltype(parity)::value;
+        bf16x8 pa[2][3], pb[2][3];
+#pragma unroll
+        for (int pp = 0; pp < 3; ++pp)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int p = pp == 0 ? 1 : pp == 1 ? 0 : 2;
+                // (32 rows further down the swizzle is the same)
+                pa[i][p] = *(const bf16x8*)(ra + P * kStageBytes + p * kPlaneBytes + i * 32 * kRowBytes);
+                pb[i][p] = *(const bf16x8*)(rb + P * kStageBytes + p * kPlaneBytes + i * 32 * kRowBytes);
+            }
+        w.a.store_cut(va[1 - P], lds + (1 - P) * kStageBytes, lost);
+        w.b.store_cut(vb[1 - P], lds + (1 - P) * kStageBytes + kOperandBytes, lost);
+        // the small products first, those whose operands are read first before the others
+        constexpr int PA[6] = {1, 0, 1, 0, 2, 0}, PB[6] = {1, 1, 0, 2, 0, 0};
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[i][PA[q]], pb[j][PB[q]], P == 0 && q == 0 ? floatx16{} : part[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+        for (int i = 0; i < 24; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (i < 8) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+            if (i >= 12 && i % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+        }
+    };
+    using Even = std::integral_constant<int, 0>;
+    using Odd = std::integral_constant<int, 1>;
+    w.fetch(g, va[0], vb[0], m0, n0);
+    w.fetch(g, va[1], vb[1], m0, n0);
+    c.settle(g, w, va[0], vb[0], m0, n0);
+    w.a.store_cut(va[0], lds, lost);
+    w.b.store_cut(vb[0], lds + kOperandBytes, lost);
+    w.fetch(g, va[0], vb[0], m0, n0);
+    lds_barrier();
+    // (behind the last slab it is cut once more, into the buffer that nobody reads again)
+    for (int s = 0; s < count; s += 2) {
+        c.settle(g, w, va[1], vb[1], m0, n0);
+        multiply(Even{});
+        w.fetch(g, va[1], vb[1], m0, n0);
+        lds_barrier();
+        c.settle(g, w, va[0], vb[0], m0, n0);
+        if (s + 1 < count) multiply(Odd{});
+        w.fetch(g, va[0], vb[0], m0, n0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] += part[i][j];
+        lds_barrier();
+    }
+
+    // a sum that is not finite, or bits below the last piece: this tile again with the fp32 instructions
+    float probe = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) probe = fmaf(acc[i][j][v], 0.0f, probe);
+        }
+    if (__syncthreads_or((lost & 0xffffu) != 0 || probe != 0.0f)) {  // (0 * x is 0 for finite x and NaN else)
+        float* la = (float*)lds;
+        float* lb = la + kTile * 17;
+        static_assert(2 * kTile * 17 * sizeof(float) <= 2 * kStageBytes, "the fp32 slab fits the pieces' LDS");
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = floatx16{};
+        w.start(g, first_term, first_k, count, m0, n0);
+        c.start(g, first_term, first_k);
+        for (int r = 0; r < count; ++r) {
+            w.fetch(g, va[0], vb[0], m0, n0);
+            c.settle(g, w, va[0], vb[0], m0, n0);
+            __syncthreads();
+            w.a.store_plain(va[0], la);
+            w.b.store_plain(vb[0], lb);
+            __syncthreads();
+            for (int k = 0; k < kSlab; k += 2) {
+                float fa[2], fb[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    fa[i] = la[(wm + 32 * i + (lane & 31)) * 17 + k + (lane >> 5)];
+                    fb[i] = lb[(wn + 32 * i + (lane & 31)) * 17 + k + (lane >> 5)];
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i], fb[j], acc[i][j], 0, 0, 0);
+            }
+        }
+    }
+
+    if (g.shares > 1) {
+        floatx4* d = (floatx4*)(g.partials + ((size_t)share * tiles + tile) * (kTile * kTile)) + tid;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) d[((i * 2 + j) * 4 + q) * 256] = floatx4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int n = n0 + wn + 32 * j + (lane & 31), m = m0 + wm + 4 * (lane >> 5);
+            if (n >= g.N) continue;
+            float* d = g.C + (size_t)m * g.ldc + n;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int r = 32 * i + 8 * (v >> 2) + (v & 3);
+                if (m + r >= g.M) continue;
+                if (g.map.on) store_result(g, m + r, n, acc[i][j][v]);
+                else put(g, d + (size_t)r * g.ldc, acc[i][j][v]);  // (the row's distance is the same for all lanes)
+            }
+        }
+}
+
+// adds the shares of a tile up in their order: a thread takes four rows of one column, sixteen workgroups a tile
+__global__ __launch_bounds__(256) void sgemm_split_fold(SplitArgs g) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, tiles = g.tiles_m * g.tiles_n;
+    const int tile = blockIdx.x >> 4, quad = blockIdx.x & 15;
+    const floatx4* p = (const floatx4*)(g.partials + (size_t)tile * (kTile * kTile)) + quad * 256 + tid;
+    const size_t pitch = (size_t)tiles * (kTile * kTile / 4);
+    floatx4 sum = p[0];
+    int s = 1;
+    for (; s + 8 <= g.shares; s += 8) {
+        floatx4 part[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) part[i] = p[(s + i) * pitch];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum += part[i];
+    }
+    for (; s < g.shares; ++s) sum += p[s * pitch];
+    const int band = tile / (8 * g.tiles_n), band_rows = min(8, g.tiles_m - 8 * band), in_band = tile - band * 8 * g.tiles_n;
+    const int tm = 8 * band + in_band % band_rows, tn = in_band / band_rows;
+    const int i = quad >> 3, j = (quad >> 2) & 1, q = quad & 3;
+    const int n = tn * kTile + 64 * (wave & 1) + 32 * j + (lane & 31);
+    const int m = tm * kTile + 64 * (wave >> 1) + 32 * i + 8 * q + 4 * (lane >> 5);
+    if (n >= g.N) return;
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+        if (m + v < g.M) store_result(g, m + v, n, sum[v]);
+}
+
+}  // namespace
+
+int sgemm_split(bool ta, bool tb, int M, int N, int nseg, const int* K, const float* const* A, const int* lda, const float* const* B, const int* ldb, float alpha,
+                float beta, float* C, int ldc, const SgemmRowMap& map, int cus) {
+    static const int enabled = getenv("DALI_HIP_GEMM_SPLIT") ? atoi(getenv("DALI_HIP_GEMM_SPLIT")) : 1;
+    // (a sum of two products keeps the order of summation that the fused LSTM step has)
+    if (!enabled || cus < 8 || nseg < 1 || nseg > kMaxTerms || nseg == 2 || M <= 64 || N <= 64 || K[0] <= 64) return 0;
+    SplitArgs g = {};
+    for (int s = 0; s < nseg; ++s) {
+        // offsets within a slab are 32-bit
+        const size_t a_span = (ta ? (size_t)kSlab * lda[s] + M : (size_t)kTile * lda[s] + kSlab), b_span = (tb ? (size_t)kTile * ldb[s] + kSlab : (size_t)kSlab * ldb[s] + N);
+        if (K[s] < kSlab || a_span >= ((size_t)1 << 30) || b_span >= ((size_t)1 << 30)) return 0;
+        g.A[s] = A[s];
+        g.B[s] = B[s];
+        g.lda[s] = lda[s];
+        g.ldb[s] = ldb[s];
+        g.K[s] = K[s];
+        g.slabs += (K[s] + kSlab - 1) / kSlab;
+    }
+    g.nseg = nseg;
+    g.M = M;
+    g.N = N;
+    g.C = C;
+    g.ldc = ldc;
+    g.alpha = alpha;
+    g.beta = beta;
+    g.map = map;
+    g.tiles_m = (M + kTile - 1) / kTile;
+    g.tiles_n = (N + kTile - 1) / kTile;
+    const long tiles = (long)g.tiles_m * g.tiles_n;
+    if (tiles > (1L << 24)) return 0;
+    // Whether and in how many shares, by estimated microseconds. Two workgroups on a compute unit pass a slab each in 1.6 us, one alone in
+    // 1.0; starting and ending a tile costs four slabs; adding shares up costs a launch and a read of them. The fp32 kernels:
+    // 112 TFLOP/s over whole 64x64 tiles, 76 where several terms or a row map leave them the register-staged kernel. Measured on both
+    // sides of the line, us here / there: [256,4096] over 2048 40 / 33, [93312,576] over 128 146 / 137, 1024^3 32 / 19 (not taken);
+    // [100352,128] over 576 124 / 131, 2048^3 112 / 130, [256,32000] over 1024 105 / 159 (taken).
+    const int most = (int)(kWorkspacePartialBytes / (kTile * kTile * sizeof(float)) / tiles);
+    auto estimate = [&](int sh) {
+        const long per_cu = (tiles * sh + cus - 1) / cus;
+        const double slabs = (double)g.slabs / sh + 4.0;
+        return (per_cu < 2 ? slabs : 0.8 * (double)per_cu * slabs) + (sh > 1 ? 4.0 + 0.013 * (double)(tiles * sh) : 0.0);
+    };
+    g.shares = 1;
+    for (int sh = 2; sh <= most && sh * 8 <= g.slabs; ++sh)
+        if (estimate(sh) < estimate(g.shares)) g.shares = sh;
+    const double fp32_rate = nseg > 2 || map.on ? 76e6 : 112e6;
+    double flops = 0.0;
+    for (int s = 0; s < nseg; ++s) flops += 2.0 * ((M + 63) / 64 * 64) * ((N + 63) / 64 * 64) * (double)K[s];
+    if (estimate(g.shares) > 0.97 * flops / fp32_rate) return 0;
+    if ((long)g.slabs * (g.shares + 1) >= (1L << 31)) return 0;
+    g.partials = (float*)(workspace() + kWorkspaceCounterBytes);
+    const dim3 grid((unsigned)(tiles * g.shares));
+    if (!ta && !tb) hipLaunchKernelGGL((sgemm_split_kernel<false, false>), grid, dim3(256), 0, stream(), g);
+    else if (ta && !tb) hipLaunchKernelGGL((sgemm_split_kernel<true, false>), grid, dim3(256), 0, stream(), g);
+    else if (!ta && tb) hipLaunchKernelGGL((sgemm_split_kernel<false, true>), grid, dim3(256), 0, stream(), g);
+    else hipLaunchKernelGGL((sgemm_split_kernel<true, true>), grid, dim3(256), 0, stream(), g);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && g.shares > 1) {
+        hipLaunchKernelGGL(sgemm_split_fold, dim3((unsigned)(tiles * 16)), dim3(256), 0, stream(), g);
+        e = hipGetLastError();
+    }
+    if (e != hipSuccess) return fail("sgemm launch failed: %s", hipGetErrorString(e));
+    return 1;
+}
+
+}  // namespace dali_hip

@@ -1,0 +1,109 @@
+"""Large fp32 products, which go through the bf16 matrix cores with every value cut in three (dali_amd/csrc/sgemm_split.hip),
+against numpy in double precision. Sizes are the smallest for which the rule in that file takes a product."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(hip, a):
+    p = C.c_void_p()
+    assert hip.dali_hip_malloc(C.byref(p), a.nbytes) == 0
+    assert hip.dali_hip_memcpy_h2d(p, a.ctypes.data_as(C.c_void_p), a.nbytes) == 0
+    return p
+
+
+def _product(hip, A, B, ta, tb, alpha=1.0, beta=0.0, pad=0, C0=None):
+    """alpha * op(A) . op(B) + beta * C0 through the column-major entry point, operands stored with `pad` NaN behind each row."""
+    K, M = A.shape if ta else A.shape[::-1]
+    N = B.shape[0] if tb else B.shape[1]
+    pa, pb = (np.ascontiguousarray(np.pad(x, ((0, 0), (0, pad)), constant_values=np.nan)) for x in (A, B))
+    out = np.full((M, N + pad), 7.0, np.float32)
+    if C0 is not None:
+        out[:, :N] = C0
+    da, db, dc = (_dev(hip, x) for x in (pa, pb, out))
+    try:
+        assert hip.dali_hip_sgemm(int(tb), int(ta), N, M, K, alpha, db, pb.shape[1], da, pa.shape[1], beta, dc, N + pad) == 0
+        assert hip.dali_hip_memcpy_d2h(out.ctypes.data_as(C.c_void_p), dc, out.nbytes) == 0
+    finally:
+        for p in (da, db, dc):
+            hip.dali_hip_free(p)
+    assert np.all(out[:, N:] == 7.0)
+    return out[:, :N]
+
+
+def _tolerance(K):
+    # Relative error in the 2-norm for operands of random sign. Each of the K / 32 additions of a chain's sum rounds a partial sum
+    # that grows as sqrt(k): together at most sqrt(K / 32) half units, and the chain itself four. (Measured: about a third.)
+    return (np.sqrt(K / 32.0) + 4.0) * 2.0 ** -24
+
+
+def _check(got, ref, K):
+    assert np.linalg.norm(got - ref) <= _tolerance(K) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+# whole tiles and slabs; a tile row with one row, a slab with one value; odd rows and a slab one short; few rows in many shares; few slabs
+@pytest.mark.parametrize("M,N,K,pad", [(2048, 2048, 2048, 0), (1985, 1923, 2049, 0), (2047, 2047, 2047, 3), (255, 1023, 30001, 1), (1023, 32001, 257, 0)])
+def test_sizes(gpu, ta, tb, M, N, K, pad):
+    rng = np.random.RandomState(M + N + K)
+    a, b = rng.randn(M, K).astype(np.float32), rng.randn(K, N).astype(np.float32)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    _check(_product(gpu, a.T.copy() if ta else a, b.T.copy() if tb else b, ta, tb, pad=pad), ref, K)
+
+
+def test_whole_numbers_are_exact_and_alpha_beta(gpu):
+    rng = np.random.RandomState(5)
+    a, b, c = (rng.randint(-31, 32, s).astype(np.float32) for s in ((2040, 2050), (2050, 2040), (2040, 2040)))
+    ref = a.astype(np.float64) @ b.astype(np.float64)  # below 2^24: every sum is exact
+    assert np.array_equal(_product(gpu, a, b, 0, 0), ref)
+    assert np.array_equal(_product(gpu, a, b, 0, 0, alpha=0.5, beta=2.0, C0=c), 0.5 * ref + 2.0 * c)
+
+
+@pytest.mark.parametrize("shape", [(2040, 2040, 2050), (200, 1000, 32000)])
+def test_values_that_three_bf16_do_not_hold(gpu, shape):
+    """Infinities, NaN, values next to the largest float and values whose last bits lie below the smallest bf16: what the fp32
+    instructions make of them."""
+    M, N, K = shape
+    rng = np.random.RandomState(6)
+    a, b = rng.randn(M, K).astype(np.float32), rng.randn(K, N).astype(np.float32)
+    a[3, 17], a[5, K - 1], a[140, 40] = np.inf, -np.inf, np.nan
+    b[K // 2, 900] = np.inf
+    a[150, :] *= np.float32(2.0 ** -125)  # denormal in part
+    a[151, :] *= np.float32(2.0 ** -112)
+    a[152, 7] = np.finfo(np.float32).max
+    b[7, :] *= np.float32(2.0 ** -20)
+    with np.errstate(all="ignore"):
+        ref = a.astype(np.float64) @ b.astype(np.float64)
+    got = _product(gpu, a, b, 0, 0)
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
+    fin = np.isfinite(ref)
+    assert np.array_equal(np.sign(got[np.isinf(ref)]), np.sign(ref[np.isinf(ref)]))
+    for m in (0, 150, 151, 152):
+        # (row 150: its sums are denormal or close to it, where a float resolves 2^-149: each of the K roundings adds half of that at most)
+        slack = 0.5 * 2.0 ** -149 * K * np.sqrt(N) if m == 150 else 0.0
+        assert np.linalg.norm((got[m] - ref[m])[fin[m]]) <= _fp32_tolerance(K) * np.linalg.norm(ref[m][fin[m]]) + slack
+
+
+def _fp32_tolerance(K):
+    # rows that the fp32 instructions sum two values of k at a time: sqrt(K / 2) half units by the same reasoning
+    return (np.sqrt(K / 2.0) + 4.0) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("fmt", ["NHWC", "NCHW"])
+@pytest.mark.parametrize("n,side,cin,cout,window", [(16, 58, 64, 128, 3), (9, 61, 67, 130, 5)])
+def test_convolution_terms_with_a_row_map(gpu, D, fmt, n, side, cin, cout, window):
+    rng = np.random.RandomState(7)
+    x = rng.randn(n, side, side, cin).astype(np.float32)
+    w = (rng.randn(cout, window, window, cin) / np.sqrt(window * window * cin)).astype(np.float32)
+    out = side - window + 1
+    ref = np.zeros((n, out, out, cout))
+    for i in range(window):
+        for j in range(window):
+            ref += x[:, i:i + out, j:j + out, :].astype(np.float64) @ w[:, i, j, :].astype(np.float64).T
+    put = (lambda t: t) if fmt == "NHWC" else (lambda t: np.ascontiguousarray(t.transpose(0, 3, 1, 2)))
+    got = D.op.conv2d(D.Array.from_numpy(put(x)), D.Array.from_numpy(put(w)), 1, 1, "valid", fmt).numpy()
+    # (not every layout takes this path at every size: the bound of the fp32 instructions)
+    assert np.linalg.norm(got - put(ref)) <= _fp32_tolerance(window * window * cin) * np.linalg.norm(ref)
