@@ -8,9 +8,13 @@
 // of weight 2^-16 and more are summed (hh, hm, mh, hl, lh, mm); those left out, ml + lm + ll, come to at most 2^-26 |a b|, a quarter of
 // what rounding one fp32 product may cost. Products of bf16 pieces are exact in fp32 and the sums are kept in fp32.
 //
-// Where the pieces do not represent the value the tile is redone with the fp32 instructions (`redo`): infinities, NaN and values that
-// round to infinity in bf16 leave a sum that is not finite; values whose last piece falls below the smallest bf16 leave
-// bits in the low half of that piece, which the cutting collects. So are tiles whose sums overflow.
+// Both operands are multiplied by 2^16 as they are cut and the sums by 2^-32 at the end: the smallest float, 2^-149, becomes the smallest
+// bf16, so that no value is too small for its pieces (the conversion and the matrix instruction keep denormal values). Without
+// that a single entry below 2^-110, as a softmax gradient has where a logit lies 76 below the largest, loses bits.
+// Infinities, NaN, values from about 2^112 and sums from 2^96 on leave a scaled sum that is not finite: such a tile is redone
+// with the fp32 instructions on the values as they are, whatever they come to. [256,1024].[1024,32000]: one entry in 61 below 2^-110
+// 99 us as without them (246 while the last piece lost bits and such tiles were redone), a NaN in every strip of rows 234
+// us, the fp32 kernels 138.
 //
 // What a MFMA of this kind adds to its accumulator is rounded more coarsely than a chain of fp32 instructions would: over a whole
 // inner extent of 512 the sums were 3.4e-7 from double precision against 1.5e-7 for the fp32 kernels. So a chain covers two slabs only
@@ -79,14 +83,17 @@ __device__ __forceinline__ unsigned int pack2(float a, float b) {
     return __builtin_bit_cast(unsigned int, __builtin_convertvector(v, bf16x2));
 }
 
-// two neighbours in k cut into their three pieces; `lost` collects what the last piece cannot hold (its low half)
-__device__ __forceinline__ void cut2(float a, float b, unsigned int& h, unsigned int& m, unsigned int& l, unsigned int& lost) {
+constexpr float kScale = 0x1p16f, kScaleBack = 0x1p-32f;  // of each operand; of the sums of products
+
+// two neighbours in k, scaled, cut into their three pieces
+__device__ __forceinline__ void cut2(float a, float b, unsigned int& h, unsigned int& m, unsigned int& l) {
+    a *= kScale;
+    b *= kScale;
     h = pack2(a, b);
     const float a1 = a - lo_part(h), b1 = b - hi_part(h);
     m = pack2(a1, b1);
     const float a2 = a1 - lo_part(m), b2 = b1 - hi_part(m);
     l = pack2(a2, b2);
-    lost |= __float_as_uint(a2) | __float_as_uint(b2);
 }
 
 __device__ __forceinline__ int lds_offset(int row, int granule) {
@@ -134,12 +141,12 @@ struct Loader {
             v[j] = k < left ? a : 0.0f;
         }
     }
-    __device__ __forceinline__ void store_cut(const float* v, char* lds, unsigned int& lost) const {
+    __device__ __forceinline__ void store_cut(const float* v, char* lds) const {
         uintx4 h, m, l;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             unsigned int hq, mq, lq;
-            cut2(v[2 * q], v[2 * q + 1], hq, mq, lq, lost);
+            cut2(v[2 * q], v[2 * q + 1], hq, mq, lq);
             h[q] = hq;
             m[q] = mq;
             l[q] = lq;
@@ -149,7 +156,7 @@ struct Loader {
         *(uintx4*)(d + kPlaneBytes) = m;
         *(uintx4*)(d + 2 * kPlaneBytes) = l;
     }
-    // as fp32, rows of 16 k and a pitch of 17 (the redo path)
+    // as fp32, rows of 16 k and a pitch of 17 (a tile that is redone)
     __device__ __forceinline__ void store_plain(const float* v, float* lds) const {
 #pragma unroll
         for (int j = 0; j < 8; ++j) lds[row * 17 + 8 * granule + j] = v[j];
@@ -274,7 +281,6 @@ __global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = floatx16{};
     const int wm = 64 * (wave >> 1), wn = 64 * (wave & 1);
-    unsigned int lost = 0;
     Walk<TA, TB> w;
     w.a.init(tid, m0, g.M, 0);
     w.b.init(tid, n0, g.N, 0);
@@ -302,8 +308,8 @@ __global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
                 pa[i][p] = *(const bf16x8*)(ra + P * kStageBytes + p * kPlaneBytes + i * 32 * kRowBytes);
                 pb[i][p] = *(const bf16x8*)(rb + P * kStageBytes + p * kPlaneBytes + i * 32 * kRowBytes);
             }
-        w.a.store_cut(va[1 - P], lds + (1 - P) * kStageBytes, lost);
-        w.b.store_cut(vb[1 - P], lds + (1 - P) * kStageBytes + kOperandBytes, lost);
+        w.a.store_cut(va[1 - P], lds + (1 - P) * kStageBytes);
+        w.b.store_cut(vb[1 - P], lds + (1 - P) * kStageBytes + kOperandBytes);
         // the small products first, those whose operands are read first before the others
         constexpr int PA[6] = {1, 0, 1, 0, 2, 0}, PB[6] = {1, 1, 0, 2, 0, 0};
 #pragma unroll
@@ -326,8 +332,8 @@ __global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
     w.fetch(g, va[0], vb[0], m0, n0);
     w.fetch(g, va[1], vb[1], m0, n0);
     c.settle(g, w, va[0], vb[0], m0, n0);
-    w.a.store_cut(va[0], lds, lost);
-    w.b.store_cut(vb[0], lds + kOperandBytes, lost);
+    w.a.store_cut(va[0], lds);
+    w.b.store_cut(vb[0], lds + kOperandBytes);
     w.fetch(g, va[0], vb[0], m0, n0);
     lds_barrier();
     // (behind the last slab it is cut once more, into the buffer that nobody reads again)
@@ -346,7 +352,7 @@ __global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
         lds_barrier();
     }
 
-    // a sum that is not finite, or bits below the last piece: this tile again with the fp32 instructions
+    // a sum that is not finite: this tile again with the fp32 instructions
     float probe = 0.0f;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -355,7 +361,7 @@ __global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) probe = fmaf(acc[i][j][v], 0.0f, probe);
         }
-    if (__syncthreads_or((lost & 0xffffu) != 0 || probe != 0.0f)) {  // (0 * x is 0 for finite x and NaN else)
+    if (__syncthreads_or(probe != 0.0f)) {  // (0 * x is 0 for finite x and NaN else)
         float* la = (float*)lds;
         float* lb = la + kTile * 17;
         static_assert(2 * kTile * 17 * sizeof(float) <= 2 * kStageBytes, "the fp32 slab fits the pieces' LDS");
@@ -365,13 +371,14 @@ __global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
             for (int j = 0; j < 2; ++j) acc[i][j] = floatx16{};
         w.start(g, first_term, first_k, count, m0, n0);
         c.start(g, first_term, first_k);
+        w.fetch(g, va[0], vb[0], m0, n0);
         for (int r = 0; r < count; ++r) {
-            w.fetch(g, va[0], vb[0], m0, n0);
             c.settle(g, w, va[0], vb[0], m0, n0);
-            __syncthreads();
+            lds_barrier();
             w.a.store_plain(va[0], la);
             w.b.store_plain(vb[0], lb);
-            __syncthreads();
+            w.fetch(g, va[0], vb[0], m0, n0);  // (in flight while this slab is multiplied)
+            lds_barrier();
             for (int k = 0; k < kSlab; k += 2) {
                 float fa[2], fb[2];
 #pragma unroll
@@ -385,6 +392,11 @@ __global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
                     for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[i], fb[j], acc[i][j], 0, 0, 0);
             }
         }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] *= kScaleBack;
     }
 
     if (g.shares > 1) {

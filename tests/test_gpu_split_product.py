@@ -92,6 +92,48 @@ def _fp32_tolerance(K):
     return (np.sqrt(K / 2.0) + 4.0) * 2.0 ** -24
 
 
+def _split_tolerance(K):
+    """Relative error in the 2-norm that the split product stays within and the fp32 kernels, two values of k at a time, do not.
+    Rounding a sum to 24 bits is off by up to half a unit, evenly: 2^-24 / sqrt(6) of it in the root mean square over its leading
+    digits. n = K / 32 chains are added to a sum whose variance grows as j / n: sqrt((n + 1) / 2) such errors together; four for
+    the chain's own roundings. Twice that."""
+    return 2.0 * 2.0 ** -24 / np.sqrt(6.0) * np.sqrt((np.ceil(K / 32.0) + 1.0) / 2.0 + 4.0)
+
+
+def _norm_ratio(got, ref):
+    return np.linalg.norm(got - ref) / np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_tiny_values_do_not_send_their_tile_to_the_fp32_instructions(gpu, ta, tb):
+    """A few entries far below the others, as a softmax gradient has them, and whole strips of rows whose pieces are denormal."""
+    M, N, K = 2048, 1920, 2050
+    rng = np.random.RandomState(8)
+    a, b = rng.randn(M, K).astype(np.float32), (rng.randn(K, N) * 2.0 ** 40).astype(np.float32)
+    a[:, 5::61] *= np.float32(2.0 ** -116)
+    powers = {128: -105, 256: -112, 384: -124, 512: -149 + 13}  # (the last: whole multiples of the smallest float)
+    for m, p in powers.items():
+        a[m:m + 128] = np.ldexp(rng.randn(128, K), p).astype(np.float32)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    got = _product(gpu, a.T.copy() if ta else a, b.T.copy() if tb else b, ta, tb)
+    for m in [0] + sorted(powers) + [640]:
+        assert _norm_ratio(got[m:m + 128], ref[m:m + 128]) <= _split_tolerance(K), m
+
+
+@pytest.mark.parametrize("bits", [(17, 2), (2, 17), (12, 7)])
+@pytest.mark.parametrize("powers", [(0, 0), (-149, 100), (100, -149), (-130, 60), (-70, -60)])
+def test_whole_numbers_of_several_pieces_are_exact(gpu, bits, powers):
+    """Whole numbers that take two or three pieces, and the same as multiples of powers of two down to the smallest float."""
+    M, N, K, chosen = 2048, 1920, 2048, 16
+    rng = np.random.RandomState(9)
+    a, b = (rng.randint(-2 ** n + 1, 2 ** n, s).astype(np.float64) for n, s in zip(bits, ((M, K), (K, N))))
+    # sixteen terms a row, so that every sum is below 2^24 and exact
+    a[~(np.argsort(rng.rand(M, K), axis=1) < chosen)] = 0.0
+    ref = np.ldexp(a @ b, powers[0] + powers[1])
+    a, b = (np.ldexp(x, p).astype(np.float32) for x, p in zip((a, b), powers))
+    assert np.array_equal(_product(gpu, a, b, 0, 0), ref.astype(np.float32))
+
+
 @pytest.mark.parametrize("fmt", ["NHWC", "NCHW"])
 @pytest.mark.parametrize("n,side,cin,cout,window", [(16, 58, 64, 128, 3), (9, 61, 67, 130, 5)])
 def test_convolution_terms_with_a_row_map(gpu, D, fmt, n, side, cin, cout, window):
