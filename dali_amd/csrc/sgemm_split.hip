@@ -3,10 +3,12 @@
 // Row-major view: C[M,N] = alpha * sum_s A_s[M,K_s] * B_s[K_s,N] + beta * C with A stored [M][K] or [K][M] and B stored [K][N] or [N][K].
 //
 // What bounds the kernels it stands in for is the fp32 matrix rate (157 TFLOP/s; a bf16 instruction does sixteen times as much per
-// cycle). With h = bf16(x), m = bf16(x - h), l = x - h - m, all rounded to nearest, x = h + m + l holds exactly: 24 significant
-// bits in three times 8, and the exponent range of bf16 is that of fp32. Of the nine products of the pieces of a and b the six
-// of weight 2^-16 and more are summed (hh, hm, mh, hl, lh, mm); those left out, ml + lm + ll, come to at most 2^-26 |a b|, a quarter of
-// what rounding one fp32 product may cost. Products of bf16 pieces are exact in fp32 and the sums are kept in fp32.
+// cycle). The cut is that of Henry, Tang and Heinecke ("Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision
+// Computations", 2019): with h = bf16(x), m = bf16(x - h), l = x - h - m, all rounded to nearest, x = h + m + l holds exactly: 24
+// significant bits in three times 8, and the exponent range of bf16 is that of fp32. Of the nine products of the pieces of a and b the six
+// of weight 2^-16 and more are summed (hh, hm, mh, hl, lh, mm). m reaches 2^-8 and l 2^-17 of the value's power of two, so those left
+// out, ml + lm + ll, come to at most 2^-24 |a b|: what rounding one fp32 product costs at most. Products of bf16 pieces are exact in
+// fp32 and the sums are kept in fp32.
 //
 // Both operands are multiplied by 2^16 as they are cut and the sums by 2^-32 at the end: the smallest float, 2^-149, becomes the smallest
 // bf16, so that no value is too small for its pieces (the conversion and the matrix instruction keep denormal values). Without
@@ -16,23 +18,28 @@
 // 99 us as without them (246 while the last piece lost bits and such tiles were redone), a NaN in every strip of rows 234
 // us, the fp32 kernels 138.
 //
-// What a MFMA of this kind adds to its accumulator is rounded more coarsely than a chain of fp32 instructions would: over a whole
-// inner extent of 512 the sums were 3.4e-7 from double precision against 1.5e-7 for the fp32 kernels. So a chain covers two slabs only
-// (32 values of k, smallest products first) and is then added to the sums by the vector unit: 1.07e-7 (normal values, K = 512;
-// K = 133: 0.83e-7 against 1.11e-7, K = 1999: 1.2e-7 against 2.1e-7, K = 32000: 2.9e-7 against 5.7e-7).
+// A MFMA of this kind cuts off (does not round) what an addend has below about 2^-25 of the largest: small products added to a large sum
+// lose their ends, over a whole inner extent and within one product alike. So the five small products have sums of their
+// own, a 2^-8 of the result, where that does not matter; hh is summed over two slabs (32 values of k) from zero and added to
+// the sums by the vector unit, as are the small ones at the end. Distance from double precision, results of [2048,2048], normal
+// operands (in brackets the fp32 kernels): K = 133 0.58e-7 (2.0e-7), 512 0.86e-7 (4.1e-7), 1999 1.2e-7 (7.9e-7); [1024,1024] over 32000 2.2e-7
+// (2.3e-6). Rows of one product only (a diagonal operand) 2.58e-8 in the root mean square and 9.9e-8 at worst (2.53e-8, 6.0e-8: an
+// fp32 product rounded once), two and more in a row already less than there. With all six in one sum a diagonal operand showed 3.3e-8 and
+// 15.7e-8; with the two largest of those left out as well, 2.53e-8 and 6.0e-8, but at 131, 144 and 130 us for the three products
+// below, which is the time of the fp32 kernels.
 //
 // A workgroup of four waves owns a 128x128 tile, a wave 64x64 of it as 2x2 accumulators of v_mfma_f32_32x32x16_bf16. Slabs of 16
-// values of k come through registers (fetched two slabs ahead), are cut there, once per workgroup and value, and written to
+// values of k come through registers (fetched one slab ahead), are cut there, once per workgroup and value, and written to
 // LDS as three planes of [row][16 k] in bf16: whatever the storage order, a lane packs neighbours in k, so the transposition of
-// [K][x] operands costs nothing. Two stages of 24 KiB, one barrier per slab: while a slab is multiplied the next one is cut. 48 KiB
-// and at most 256 registers: two workgroups share a compute unit.
+// [K][x] operands costs nothing. m and l have two stages, h a ring of four: while a slab is multiplied the next one is cut, and the second
+// slab of a pair finds h of the first. One barrier per slab. 64 KiB and at most 256 registers: two workgroups share a compute unit.
 //
-// Measured (random operands): [256,1024].[1024,32000] 159 -> 105 us, its gradients [1024,256].[256,32000] 149 -> 123 us and
-// [256,32000].[32000,1024] 146 -> 104 us; 4096^3 with B stored [N][K] 950 -> 740 us (186 TFLOP/s), [K][N] 970 -> 884 us. The matrix instructions alone take
-// 490 us of that (the card holds about 1.75 GHz under them); cutting and writing to LDS is what does not hide behind them: with one
-// of the six products 390 us, without cutting 640. Measured and dropped: separate sums for the small products (no more accurate and
-// no faster), slabs of 32 with two barriers, three stages with operands read ahead of the barrier (790 us), subtracting with
-// v_dot2_f32_bf16 (slower and not exact).
+// Measured (normal operands): [256,1024].[1024,32000] 145 -> 116 us, its gradients [1024,256].[256,32000] 130 -> 123 us and
+// [256,32000].[32000,1024] 129 -> 107 us; 4096^3 943 -> 769 us, with B stored [N][K] 948 -> 757, A stored [K][M] 925 -> 770, both 946 -> 768.
+// The matrix instructions alone take about 490 us of that (the card holds about 1.75 GHz under them); cutting, adding and writing to LDS is what
+// does not hide behind them. Measured and dropped: all six products in one sum, added every 32 k (735 us, and the loss above),
+// slabs of 32 with two barriers, fetching two slabs ahead (no faster, registers), subtracting with v_dot2_f32_bf16 (slower and not
+// exact).
 //
 // LDS rows are 32 bytes, two 16-byte granules of eight k. Granule g of row r lies in slot g ^ (bit 2 of r) of the row whose bit 2 is
 // flipped where bit 3 of r is set: eight neighbouring rows touch eight different 16-byte columns of 128 bytes, sixteen touch sixteen of
@@ -57,8 +64,9 @@ typedef floatx4 floatx4u __attribute__((aligned(4)));
 constexpr int kTile = 128, kSlab = 16;
 constexpr int kRowBytes = kSlab * 2;
 constexpr int kPlaneBytes = kTile * kSlab * 2;     // one piece of one operand
-constexpr int kOperandBytes = 3 * kPlaneBytes;
-constexpr int kStageBytes = 2 * kOperandBytes;     // the pieces of one slab of both operands; two stages
+constexpr int kHighBytes = 2 * kPlaneBytes;        // h of one slab of both operands: a ring of four slabs
+constexpr int kLowBytes = 4 * kPlaneBytes;         // m and l: two stages behind the ring
+constexpr int kLow = 4 * kHighBytes, kLdsBytes = kLow + 2 * kLowBytes;
 constexpr int kMaxTerms = 8;
 
 struct SplitArgs {
@@ -141,20 +149,23 @@ struct Loader {
             v[j] = k < left ? a : 0.0f;
         }
     }
-    __device__ __forceinline__ void store_cut(const float* v, char* lds) const {
-        uintx4 h, m, l;
+    // two of the four pairs of neighbours of `v`
+    __device__ __forceinline__ static void cut_half(const float* v, int half, uintx4& h, uintx4& m, uintx4& l) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 2 * half; q < 2 * half + 2; ++q) {
             unsigned int hq, mq, lq;
             cut2(v[2 * q], v[2 * q + 1], hq, mq, lq);
             h[q] = hq;
             m[q] = mq;
             l[q] = lq;
         }
-        char* d = lds + lds_offset(row, granule);
-        *(uintx4*)d = h;
-        *(uintx4*)(d + kPlaneBytes) = m;
-        *(uintx4*)(d + 2 * kPlaneBytes) = l;
+    }
+    // `high`, `low`: this operand's planes of the slab
+    __device__ __forceinline__ void store(uintx4 h, uintx4 m, uintx4 l, char* high, char* low) const {
+        const int d = lds_offset(row, granule);
+        *(uintx4*)(high + d) = h;
+        *(uintx4*)(low + d) = m;
+        *(uintx4*)(low + d + kPlaneBytes) = l;
     }
     // as fp32, rows of 16 k and a pitch of 17 (a tile that is redone)
     __device__ __forceinline__ void store_plain(const float* v, float* lds) const {
@@ -257,7 +268,7 @@ __device__ __forceinline__ void store_result(const SplitArgs& g, int m, int n, f
 
 template <bool TA, bool TB>
 __global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
-    __shared__ __attribute__((aligned(16))) char lds[2 * kStageBytes];
+    __shared__ __attribute__((aligned(16))) char lds[kLdsBytes];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // Every eighth workgroup runs on the same die: a die takes a run of neighbouring tiles (of one share), eight rows of tiles to
     // a band, and finds the operands its other workgroups asked for in its L2.
@@ -275,11 +286,11 @@ __global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
     const int m0 = tm * kTile, n0 = tn * kTile;
     const int s_begin = uniform(g.slabs * share / g.shares), s_end = uniform(g.slabs * (share + 1) / g.shares);
 
-    floatx16 acc[2][2], part[2][2];  // the sums; those of the pair of slabs at hand
+    floatx16 acc[2][2], small[2][2];  // the sums of hh; of the other products
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = floatx16{};
+        for (int j = 0; j < 2; ++j) acc[i][j] = small[i][j] = floatx16{};
     const int wm = 64 * (wave >> 1), wn = 64 * (wave & 1);
     Walk<TA, TB> w;
     w.a.init(tid, m0, g.M, 0);
@@ -291,66 +302,91 @@ __global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
     w.start(g, first_term, first_k, count, m0, n0);
     Cutter<TA, TB> c;
     c.start(g, first_term, first_k);
-    float va[2][8], vb[2][8];  // slabs of even and odd number (counted from s_begin)
-    const char* ra = lds + lds_offset(wm + (lane & 31), lane >> 5);
-    const char* rb = lds + kOperandBytes + lds_offset(wn + (lane & 31), lane >> 5);
-
-    // slab `P` (its parity) from LDS through the matrix instructions; meanwhile the next one is cut and written to the other buffer
+    float va[8], vb[8];
+    const int ra = lds_offset(wm + (lane & 31), lane >> 5), rb = lds_offset(wn + (lane & 31), lane >> 5) + kPlaneBytes;
+    // operand fragments of the wave: A and B in turn (32 rows further down the swizzle is the same)
+    auto read = [&](bf16x8* a, bf16x8* b, const char* from, int b_off) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            a[i] = *(const bf16x8*)(from + ra + i * 32 * kRowBytes);
+            b[i] = *(const bf16x8*)(from + rb + b_off + i * 32 * kRowBytes);
+        }
+    };
+    auto mfma = [](bf16x8 a, bf16x8 b, floatx16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); };
+    int ring = 0;  // where in the ring the pair of slabs at hand begins
+    // The small products of slab `P` (its parity) of a pair, for the second also hh of both; meanwhile the next slab is cut and
+    // written to LDS. Four groups, so that no more than one sum of hh is held at a time.
     auto multiply = [&](auto parity) {
         constexpr int P = decltype(parity)::value;
-        bf16x8 pa[2][3], pb[2][3];
+        const char *high = lds + ring, *low = lds + kLow + P * kLowBytes;
+        bf16x8 ea[2], eb[2], pa[3][2], pb[3][2];  // h of the pair's first slab; h, m, l of this one
+        read(pa[0], pb[0], high + P * kHighBytes, 0);
+        read(pa[1], pb[1], low, kPlaneBytes);
+        if (P == 1) read(ea, eb, high, 0);
+        constexpr int PA[5] = {0, 1, 1, 0, 2}, PB[5] = {1, 0, 1, 2, 0};
+        char *high_to = P == 0 ? lds + ring + kHighBytes : lds + (ring ^ (2 * kHighBytes)), *low_to = lds + kLow + (1 - P) * kLowBytes;
+        uintx4 ch, cm, cl;
 #pragma unroll
-        for (int pp = 0; pp < 3; ++pp)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int p = pp == 0 ? 1 : pp == 1 ? 0 : 2;
-                // (32 rows further down the swizzle is the same)
-                pa[i][p] = *(const bf16x8*)(ra + P * kStageBytes + p * kPlaneBytes + i * 32 * kRowBytes);
-                pb[i][p] = *(const bf16x8*)(rb + P * kStageBytes + p * kPlaneBytes + i * 32 * kRowBytes);
+        for (int group = 0; group < 4; ++group) {
+            const int bi = group >> 1, bj = group & 1;
+            if (group == 1) read(pa[2], pb[2], low + kPlaneBytes, kPlaneBytes);
+            floatx16 big;
+            if (P == 1) {
+                big = mfma(ea[bi], eb[bj], floatx16{});
+                big = mfma(pa[0][bi], pb[0][bj], big);
             }
-        w.a.store_cut(va[1 - P], lds + (1 - P) * kStageBytes);
-        w.b.store_cut(vb[1 - P], lds + (1 - P) * kStageBytes + kOperandBytes);
-        // the small products first, those whose operands are read first before the others
-        constexpr int PA[6] = {1, 0, 1, 0, 2, 0}, PB[6] = {1, 1, 0, 2, 0, 0};
 #pragma unroll
-        for (int q = 0; q < 6; ++q)
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) part[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[i][PA[q]], pb[j][PB[q]], P == 0 && q == 0 ? floatx16{} : part[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
-#pragma unroll
-        for (int i = 0; i < 24; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (i < 8) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
-            if (i >= 12 && i % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+            for (int x = 5 * group; x < 5 * group + 5; ++x) {
+                const int q = x >> 2, i = (x >> 1) & 1, j = x & 1;
+                small[i][j] = mfma(pa[PA[q]][i], pb[PB[q]][j], small[i][j]);
+            }
+            Loader<TB>::cut_half(group < 2 ? va : vb, group & 1, ch, cm, cl);
+            if (group == 1) w.a.store(ch, cm, cl, high_to, low_to);
+            if (group == 3) w.b.store(ch, cm, cl, high_to + kPlaneBytes, low_to + 2 * kPlaneBytes);
+            if (P == 1) acc[bi][bj] += big;
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
     using Even = std::integral_constant<int, 0>;
     using Odd = std::integral_constant<int, 1>;
-    w.fetch(g, va[0], vb[0], m0, n0);
-    w.fetch(g, va[1], vb[1], m0, n0);
-    c.settle(g, w, va[0], vb[0], m0, n0);
-    w.a.store_cut(va[0], lds);
-    w.b.store_cut(vb[0], lds + kOperandBytes);
-    w.fetch(g, va[0], vb[0], m0, n0);
-    lds_barrier();
-    // (behind the last slab it is cut once more, into the buffer that nobody reads again)
-    for (int s = 0; s < count; s += 2) {
-        c.settle(g, w, va[1], vb[1], m0, n0);
-        multiply(Even{});
-        w.fetch(g, va[1], vb[1], m0, n0);
-        lds_barrier();
-        c.settle(g, w, va[0], vb[0], m0, n0);
-        if (s + 1 < count) multiply(Odd{});
-        w.fetch(g, va[0], vb[0], m0, n0);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] += part[i][j];
-        lds_barrier();
+    w.fetch(g, va, vb, m0, n0);
+    c.settle(g, w, va, vb, m0, n0);
+    {
+        uintx4 h, m, l;
+        Loader<TB>::cut_half(va, 0, h, m, l);
+        Loader<TB>::cut_half(va, 1, h, m, l);
+        w.a.store(h, m, l, lds, lds + kLow);
+        Loader<TB>::cut_half(vb, 0, h, m, l);
+        Loader<TB>::cut_half(vb, 1, h, m, l);
+        w.b.store(h, m, l, lds + kPlaneBytes, lds + kLow + 2 * kPlaneBytes);
     }
+    w.fetch(g, va, vb, m0, n0);
+    lds_barrier();
+    // (behind the last slab it is cut once more, to where nobody reads it again)
+    for (int s = 0; s < count; s += 2) {
+        c.settle(g, w, va, vb, m0, n0);
+        multiply(Even{});
+        w.fetch(g, va, vb, m0, n0);
+        lds_barrier();
+        if (s + 1 < count) {
+            c.settle(g, w, va, vb, m0, n0);
+            multiply(Odd{});
+            w.fetch(g, va, vb, m0, n0);
+            lds_barrier();
+        } else {
+            bf16x8 a[2], b[2];
+            read(a, b, lds + ring, 0);
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] += mfma(a[i], b[j], floatx16{});
+        }
+        ring ^= 2 * kHighBytes;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] += small[i][j];
 
     // a sum that is not finite: this tile again with the fp32 instructions
     float probe = 0.0f;
@@ -364,20 +400,20 @@ __global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
     if (__syncthreads_or(probe != 0.0f)) {  // (0 * x is 0 for finite x and NaN else)
         float* la = (float*)lds;
         float* lb = la + kTile * 17;
-        static_assert(2 * kTile * 17 * sizeof(float) <= 2 * kStageBytes, "the fp32 slab fits the pieces' LDS");
+        static_assert(2 * kTile * 17 * sizeof(float) <= kLdsBytes, "the fp32 slab fits the pieces' LDS");
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) acc[i][j] = floatx16{};
         w.start(g, first_term, first_k, count, m0, n0);
         c.start(g, first_term, first_k);
-        w.fetch(g, va[0], vb[0], m0, n0);
+        w.fetch(g, va, vb, m0, n0);
         for (int r = 0; r < count; ++r) {
-            c.settle(g, w, va[0], vb[0], m0, n0);
+            c.settle(g, w, va, vb, m0, n0);
             lds_barrier();
-            w.a.store_plain(va[0], la);
-            w.b.store_plain(vb[0], lb);
-            w.fetch(g, va[0], vb[0], m0, n0);  // (in flight while this slab is multiplied)
+            w.a.store_plain(va, la);
+            w.b.store_plain(vb, lb);
+            w.fetch(g, va, vb, m0, n0);  // (in flight while this slab is multiplied)
             lds_barrier();
             for (int k = 0; k < kSlab; k += 2) {
                 float fa[2], fb[2];

@@ -209,6 +209,10 @@ int dali_hip_cache_warm(int* loaded);
  * straight from memory into the matrix instruction, instead of being tiled through LDS; the sums are then formed in
  * another order than the tiled kernels form them (DALI_HIP_GEMM_SKINNY=0 switches this off). With k <= 64 against a
  * large C (transB = 0) the rows of A stay in registers and C is written once (DALI_HIP_GEMM_SMALLK=0 switches that off).
+ * Large products (m, n, k > 64, some 10 GFLOP and more) run on the bf16 matrix cores, every value cut into three bf16 pieces that
+ * add up to it (DALI_HIP_GEMM_SPLIT=0 switches that off). Sums of many terms come out closer to double precision than on the fp32
+ * instructions; a sum of one term only (a diagonal operand) is within one unit in the last place instead of half a one, and exact
+ * where a factor is a power of two. Infinities, NaN and overflow come out as on the fp32 instructions, in about twice the time.
  */
 int dali_hip_sgemm(int transB, int transA, int m, int n, int k, float alpha, const float* B, int ldb,
                    const float* A, int lda, float beta, float* C, int ldc);

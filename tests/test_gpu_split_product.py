@@ -105,6 +105,47 @@ def _norm_ratio(got, ref):
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("M,N,K", [(4000, 3999, 512), (4097, 2999, 1025), (2000, 4001, 2041)])
+def test_accuracy(gpu, ta, tb, M, N, K):
+    """Closer to double precision than the fp32 kernels come: also that it was this path that was taken."""
+    rng = np.random.RandomState(M + N + K)
+    a, b = rng.randn(M, K).astype(np.float32), rng.randn(K, N).astype(np.float32)
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    got = _product(gpu, a.T.copy() if ta else a, b.T.copy() if tb else b, ta, tb)
+    assert _norm_ratio(got, ref) <= _split_tolerance(K)
+    got = _product(gpu, a.T.copy() if ta else a, b.T.copy() if tb else b, ta, tb, alpha=-0.5, beta=1.0, C0=np.float32(ref))
+    # (alpha * sum + beta * C: C0 is rounded once, and so is the result, which is half as large)
+    assert _norm_ratio(got, 0.5 * ref) <= _split_tolerance(K) + 3 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_single_products(gpu, ta, tb):
+    """A diagonal left operand, mantissas at random: every result is one product. ml + lm + ll, which is left out, is at most
+    (2^-24 + 2^-34) |a b|, the last rounding at most 2^-24, and the five sums of small products (below 2^-6 |a b|) lose at most a unit each."""
+    M = N = K = 2048
+    rng = np.random.RandomState(10)
+    values = lambda *s: ((1.0 + rng.rand(*s)) * np.where(rng.rand(*s) < 0.5, -1.0, 1.0)).astype(np.float32)
+    a, b = np.diag(values(M)), values(K, N)
+    ref = np.diag(a).astype(np.float64)[:, None] * b.astype(np.float64)
+    got = _product(gpu, a, b.T.copy() if tb else b, ta, tb)
+    assert np.max(np.abs(got - ref) / np.abs(ref)) <= 2.0 ** -23 + 2.0 ** -34 + 5 * 2.0 ** -29
+    # In the 2-norm: the rounding of a product of such values, 2.49e-8, and what is left out. m is even over 2^-8 and l over 2^-17 in
+    # either direction: ml and lm 2^-25 / 3 each, over values of 7 / 3 in the root mean square. A twentieth more.
+    assert _norm_ratio(got, ref) <= 1.05 * np.hypot(2.49e-8, np.sqrt(2.0) * 2.0 ** -25 / 3.0 / (7.0 / 3.0))
+    # one operand a power of two: nothing is left out and nothing rounded
+    a = np.diag(np.ldexp(1.0, rng.randint(-60, 60, M)).astype(np.float32))
+    assert np.array_equal(_product(gpu, a, b.T.copy() if tb else b, ta, tb), np.diag(a)[:, None] * b)
+
+
+def test_equal_operands(gpu):
+    """What is left out of every product is largest, and of the same sign, for this value: 2^-24 of the sum."""
+    M, N, K = 2048, 1920, 2048
+    c = np.float32(1.0 + 2.0 ** -8 - 2.0 ** -17)
+    got = _product(gpu, np.full((M, K), c), np.full((K, N), c), 0, 0)
+    assert np.max(np.abs(got / (K * np.float64(c) ** 2) - 1.0)) <= 2.0 ** -24 + _split_tolerance(K)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 def test_tiny_values_do_not_send_their_tile_to_the_fp32_instructions(gpu, ta, tb):
     """A few entries far below the others, as a softmax gradient has them, and whole strips of rows whose pieces are denormal."""
     M, N, K = 2048, 1920, 2050
