@@ -494,7 +494,8 @@ __global__ __launch_bounds__(256) void sgemm_split_fold(SplitArgs g) {
 int sgemm_split(bool ta, bool tb, int M, int N, int nseg, const int* K, const float* const* A, const int* lda, const float* const* B, const int* ldb, float alpha,
                 float beta, float* C, int ldc, const SgemmRowMap& map, int cus) {
     static const int enabled = getenv("DALI_HIP_GEMM_SPLIT") ? atoi(getenv("DALI_HIP_GEMM_SPLIT")) : 1;
-    // (a sum of two products keeps the order of summation that the fused LSTM step has)
+    // (A sum of two products keeps the order of summation that the fused LSTM step has. What a pair stands for is not known here: two large
+    // products that have nothing to do with a cell, or two filter rows of a convolution, stay on the fp32 kernels with it.)
     if (!enabled || cus < 8 || nseg < 1 || nseg > kMaxTerms || nseg == 2 || M <= 64 || N <= 64 || K[0] <= 64) return 0;
     SplitArgs g = {};
     for (int s = 0; s < nseg; ++s) {
@@ -520,11 +521,20 @@ int sgemm_split(bool ta, bool tb, int M, int N, int nseg, const int* K, const fl
     g.tiles_n = (N + kTile - 1) / kTile;
     const long tiles = (long)g.tiles_m * g.tiles_n;
     if (tiles > (1L << 24)) return 0;
-    // Whether and in how many shares, by estimated microseconds. Two workgroups on a compute unit pass a slab each in 1.6 us, one alone in
-    // 1.0; starting and ending a tile costs four slabs; adding shares up costs a launch and a read of them. The fp32 kernels:
-    // 112 TFLOP/s over whole 64x64 tiles, 76 where several terms or a row map leave them the register-staged kernel. Measured on both
-    // sides of the line, us here / there: [256,4096] over 2048 40 / 33, [93312,576] over 128 146 / 137, 1024^3 32 / 19 (not taken);
-    // [100352,128] over 576 124 / 131, 2048^3 112 / 130, [256,32000] over 1024 105 / 159 (taken).
+    // Whether and in how many shares, by estimated microseconds. Workgroups that share a compute unit pass a slab each in 0.8 us, one alone in
+    // 1.0; starting and ending a tile costs four slabs; adding shares up costs a launch and a read of them. The fp32 kernels by their
+    // rate over whole 64x64 tiles, in TFLOP/s: 76 where several terms or a row map leave them the register-staged kernel (measured 68 to 94); 135
+    // where their loads write LDS and up to four rounds of 64x64 tiles fill the chip (117 to 141); 115 over long inner extents, where they
+    // cut what does not fill a round into shares (117 to 136 at 1.4 to 2.4 tiles a compute unit); 112 else (45 to 145: operands off 16 bytes and rounds
+    // that are not full are the slow ones). Measured, us here / there, in the orders NN NT TN TT:
+    //   one 128x128 tile a compute unit, refused: 2048^2 over 512 39 38 40 38 / 37 36 35 36, over 1024 69 68 69 67 / 65 65 63 64; 1024^2 over 4096
+    //     63 62 63 63 / 64 61 63 61; [1883,10136] against [4486,10136] (NT) 1485 / 1411; [256,4096] over 512 24 24 24 24 / 11 11 11 11
+    //   two: [2048,4096] over 256 35 34 35 35 / 37 38 36 38, over 1024 107 105 106 106 / 124 126 122 125
+    //   three: [3072,4096] over 256 52 51 52 51 / 53 54 53 54, over 1024 161 160 163 160 / 185 185 180 185, over 4096 605 599 612 598 / 711 713 698 713
+    //   five: [4096,5120] over 256 79 78 80 79 / 87 88 85 87, over 1024 260 254 260 256 / 310 311 301 309
+    //   2.4 tiles, off 16 bytes: [573,15415] over 2683 395 397 400 396 / 581 589 910 900
+    //   shares: [256,1024] over 32000 110 108 110 110 / 131 129 132 129; [576,128] over 93312 116 114 108 110 / 118 116 119 116
+    //   rows of a convolution: [100352,128] over 3 x 192 122 / 166, [3136,256] over 3 x 384 30 / 27 (refused)
     const int most = (int)(kWorkspacePartialBytes / (kTile * kTile * sizeof(float)) / tiles);
     auto estimate = [&](int sh) {
         const long per_cu = (tiles * sh + cus - 1) / cus;
@@ -534,7 +544,11 @@ int sgemm_split(bool ta, bool tb, int M, int N, int nseg, const int* K, const fl
     g.shares = 1;
     for (int sh = 2; sh <= most && sh * 8 <= g.slabs; ++sh)
         if (estimate(sh) < estimate(g.shares)) g.shares = sh;
-    const double fp32_rate = nseg > 2 || map.on ? 76e6 : 112e6;
+    bool direct = true;  // the loads of the fp32 kernels can write LDS
+    for (int s = 0; s < nseg; ++s) direct = direct && lda[s] % 4 == 0 && ldb[s] % 4 == 0 && (((uintptr_t)A[s] | (uintptr_t)B[s]) & 15) == 0;
+    const long tiles64 = (long)((M + 63) / 64) * ((N + 63) / 64), rounds64 = (tiles64 + cus - 1) / cus;
+    const bool fills = tiles <= cus && (double)tiles64 >= 0.95 * (double)(rounds64 * cus);
+    const double fp32_rate = nseg > 2 || map.on ? 76e6 : !direct ? 112e6 : fills ? 135e6 : g.shares == 1 && K[0] >= 2048 ? 115e6 : 112e6;
     double flops = 0.0;
     for (int s = 0; s < nseg; ++s) flops += 2.0 * ((M + 63) / 64 * 64) * ((N + 63) / 64 * 64) * (double)K[s];
     if (estimate(g.shares) > 0.97 * flops / fp32_rate) return 0;

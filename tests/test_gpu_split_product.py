@@ -1,6 +1,9 @@
 """Large fp32 products, which go through the bf16 matrix cores with every value cut in three (dali_amd/csrc/sgemm_split.hip),
-against numpy in double precision. Sizes are the smallest for which the rule in that file takes a product."""
+against numpy in double precision."""
 import ctypes as C
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -190,3 +193,66 @@ def test_convolution_terms_with_a_row_map(gpu, D, fmt, n, side, cin, cout, windo
     got = D.op.conv2d(D.Array.from_numpy(put(x)), D.Array.from_numpy(put(w)), 1, 1, "valid", fmt).numpy()
     # (not every layout takes this path at every size: the bound of the fp32 instructions)
     assert np.linalg.norm(got - put(ref)) <= _fp32_tolerance(window * window * cin) * np.linalg.norm(ref)
+
+
+# (ta, tb, M, N, K, elements behind each row, whether the split product takes it): on either side of the rule's lines
+_ROUTES = [
+    (0, 0, 2048, 2048, 1024, 0, False), (1, 0, 2048, 2048, 512, 0, False), (0, 1, 1024, 1024, 4096, 0, False),  # the fp32 kernels' tiles fill the chip
+    (0, 0, 2048, 2048, 4096, 0, True), (0, 1, 2048, 4096, 512, 0, True),
+    (0, 0, 2048, 2048, 1024, 1, True),                                # their loads cannot write LDS
+    (0, 1, 1920, 4096, 1030, 1, True), (0, 0, 1000, 1000, 1000, 0, False),
+    (0, 0, 3072, 4096, 1024, 0, True), (1, 0, 4096, 5120, 256, 0, True), (1, 1, 3072, 4096, 256, 0, True),  # three and five tiles a compute unit
+    (0, 0, 200, 1000, 16000, 0, True), (0, 0, 256, 4096, 1024, 0, False),  # shares
+    (0, 0, 64, 32000, 1024, 0, False), (0, 0, 4096, 4096, 64, 0, False),
+]
+# products that the kernel walking lists of 128x128 tiles had before; with the switch off it still has them
+_WALKED = [(1, 0, 1024, 32000, 256, 4), (0, 0, 4096, 768, 2048, 4), (0, 1, 8192, 1024, 320, 4), (0, 0, 3072, 1536, 1024, 4), (1, 0, 1536, 2048, 544, 4),
+           (0, 1, 3000, 1540, 416, 4), (0, 0, 768, 4096, 2048, 4), (1, 1, 2304, 2560, 2068, 4)]
+
+
+def _case_product(hip, ta, tb, M, N, K, pad):
+    rng = np.random.RandomState(M + 3 * N + 7 * K)
+    a, b = rng.randn(M, K).astype(np.float32), rng.randn(K, N).astype(np.float32)
+    return _product(hip, a.T.copy() if ta else a, b.T.copy() if tb else b, ta, tb, pad=pad), a, b
+
+
+def fp32_products(path):
+    """Run in a process that has DALI_HIP_GEMM_SPLIT=0."""
+    from dali_amd._native import hip, hip_check
+    hip_check(hip.dali_hip_init(0), "dali_hip_init")
+    for i, case in enumerate([c[:6] for c in _ROUTES] + _WALKED):
+        np.save(os.path.join(path, "%d.npy" % i), _case_product(hip, *case)[0])
+        print(case, flush=True)
+
+
+@pytest.fixture(scope="module")
+def fp32_path(gpu, tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("fp32_products"))
+    here = os.path.dirname(os.path.abspath(__file__))
+    code = "import sys; sys.path[:0] = %r; import test_gpu_split_product as t; t.fp32_products(%r)" % ([os.path.dirname(here), here], path)
+    out = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, DALI_HIP_GEMM_SPLIT="0"), stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=100)
+    assert out.returncode == 0, out.stdout
+    return path
+
+
+@pytest.mark.parametrize("i", range(len(_ROUTES)), ids=["-".join(map(str, c)) for c in _ROUTES])
+def test_which_products_are_split(gpu, fp32_path, i):
+    """A product that stays on the fp32 kernels has the bits that it has with the switch off; one that is split has others, and is
+    closer to double precision."""
+    got, a, b = _case_product(gpu, *_ROUTES[i][:6])
+    fp32 = np.load(os.path.join(fp32_path, "%d.npy" % i))
+    assert np.array_equal(got, fp32) != _ROUTES[i][6]
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    assert _norm_ratio(fp32, ref) <= _fp32_tolerance(_ROUTES[i][4])
+    if _ROUTES[i][6]:
+        assert _norm_ratio(got, ref) < _norm_ratio(fp32, ref) and _norm_ratio(got, ref) <= _split_tolerance(_ROUTES[i][4])
+
+
+@pytest.mark.parametrize("i", range(len(_WALKED)), ids=["-".join(map(str, c)) for c in _WALKED])
+def test_products_of_the_tile_walking_kernel_with_the_switch_off(gpu, fp32_path, i):
+    ta, tb, M, N, K, pad = _WALKED[i]
+    got, a, b = _case_product(gpu, *_WALKED[i])
+    fp32 = np.load(os.path.join(fp32_path, "%d.npy" % (len(_ROUTES) + i)))
+    ref = a.astype(np.float64) @ b.astype(np.float64)
+    assert _norm_ratio(fp32, ref) <= _fp32_tolerance(K)
+    assert _norm_ratio(got, ref) <= _fp32_tolerance(K)
