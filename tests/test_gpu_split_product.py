@@ -195,6 +195,67 @@ def test_convolution_terms_with_a_row_map(gpu, D, fmt, n, side, cin, cout, windo
     assert np.linalg.norm(got - put(ref)) <= _fp32_tolerance(window * window * cin) * np.linalg.norm(ref)
 
 
+def _check_specials(got, ref, K):
+    """`ref` in double precision, or what the fp32 instructions make of sums that overflow there."""
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
+    assert np.array_equal(np.sign(got[np.isinf(ref)]), np.sign(ref[np.isinf(ref)]))
+    fin = np.isfinite(ref)
+    assert np.linalg.norm(got[fin] - ref[fin]) <= _fp32_tolerance(K) * np.linalg.norm(ref[fin])
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("shape", [(2040, 4000, 1030), (200, 1000, 32007)])  # the second in shares
+@pytest.mark.parametrize("alpha,beta", [(1.0, 0.0), (-2.0, 0.5)])
+def test_tiles_redone_with_the_fp32_instructions(gpu, ta, tb, shape, alpha, beta):
+    M, N, K = shape
+    rng = np.random.RandomState(11)
+    a, b, c = (rng.randn(*s).astype(np.float32) for s in ((M, K), (K, N), (M, N)))
+    a[3, K - 1], a[5, 40], a[140, K - 9], a[M - 1, K // 2] = np.inf, -np.inf, np.nan, np.float32(2.0 ** 114)
+    b[K // 3, N - 2] = -np.inf
+    b[K // 2, 130] = np.float32(2.0 ** 13)  # 2^127 in the corner of its tile
+    with np.errstate(all="ignore"):
+        ref = alpha * (a.astype(np.float64) @ b.astype(np.float64)) + beta * c.astype(np.float64)
+        ref = np.where(np.abs(ref) >= 2.0 ** 128, np.copysign(np.inf, ref), ref)
+    got = _product(gpu, a.T.copy() if ta else a, b.T.copy() if tb else b, ta, tb, alpha, beta, pad=1, C0=c)
+    for rows in (slice(0, 128), slice(128, M - 1), slice(M - 1, M)):
+        _check_specials(got[rows], ref[rows], K)
+
+
+def test_convolution_accuracy(gpu, D):
+    """As test_accuracy: closer to double precision than the kernel that the fp32 instructions have for several terms."""
+    n, side, cin, cout, window = 16, 58, 64, 128, 3
+    rng = np.random.RandomState(13)
+    x, w = rng.randn(n, side, side, cin).astype(np.float32), rng.randn(cout, window, window, cin).astype(np.float32)
+    out = side - window + 1
+    ref = np.zeros((n, out, out, cout))
+    for i in range(window):
+        for j in range(window):
+            ref += x[:, i:i + out, j:j + out, :].astype(np.float64) @ w[:, i, j, :].astype(np.float64).T
+    got = D.op.conv2d(D.Array.from_numpy(x), D.Array.from_numpy(w), 1, 1, "valid", "NHWC").numpy()
+    assert _norm_ratio(got, ref) <= _split_tolerance(window * window * cin)
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan, 2.0 ** 120, 2.0 ** -130])
+def test_convolution_of_special_values(gpu, D, value):
+    """Three terms with overlapping rows and a row map: tiles that are redone walk the same terms; tiny values need none."""
+    n, side, cin, cout, window = 16, 58, 64, 128, 3
+    rng = np.random.RandomState(12)
+    x = rng.randn(n, side, side, cin).astype(np.float32)
+    for at in ((0, 0, 0, 0), (3, 20, 31, 7), (9, 57, 57, 63), (15, 56, 2, 30)):
+        x[at] = value
+    w = (rng.randn(cout, window, window, cin) / np.sqrt(window * window * cin)).astype(np.float32)
+    out = side - window + 1
+    ref = np.zeros((n, out, out, cout))
+    with np.errstate(all="ignore"):
+        for i in range(window):
+            for j in range(window):
+                ref += x[:, i:i + out, j:j + out, :].astype(np.float64) @ w[:, i, j, :].astype(np.float64).T
+    got = D.op.conv2d(D.Array.from_numpy(x), D.Array.from_numpy(w), 1, 1, "valid", "NHWC").numpy()
+    ordinary = np.abs(ref) < 2.0 ** 60  # (NaN is not)
+    _check_specials(got[~ordinary], ref[~ordinary], window * window * cin)
+    assert _norm_ratio(got[ordinary], ref[ordinary]) <= _fp32_tolerance(window * window * cin)
+
+
 # (ta, tb, M, N, K, elements behind each row, whether the split product takes it): on either side of the rule's lines
 _ROUTES = [
     (0, 0, 2048, 2048, 1024, 0, False), (1, 0, 2048, 2048, 512, 0, False), (0, 1, 1024, 1024, 4096, 0, False),  # the fp32 kernels' tiles fill the chip
