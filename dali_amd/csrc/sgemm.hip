@@ -1023,7 +1023,7 @@ static int sgemm_rowmajor(int nseg, bool ta, bool tb, int M, int N, const int* K
     }
     if (g.seg[0].K > 0) {
         // large products through the bf16 matrix cores: six products of the pieces of values cut in three take less time there than
-        // the one product on the fp32 ones ([256,32000] over K = 1024: 105 against 159 us; the sizes are judged there)
+        // the one product on the fp32 ones ([256,32000] over K = 1024: 116 against 145 us; the sizes are judged there)
         const float* as[kMaxSeg];
         const float* bs[kMaxSeg];
         int ks[kMaxSeg], las[kMaxSeg], lbs[kMaxSeg];

@@ -34,12 +34,13 @@
 // [K][x] operands costs nothing. m and l have two stages, h a ring of four: while a slab is multiplied the next one is cut, and the second
 // slab of a pair finds h of the first. One barrier per slab. 64 KiB and at most 256 registers: two workgroups share a compute unit.
 //
-// Measured (normal operands): [256,1024].[1024,32000] 145 -> 116 us, its gradients [1024,256].[256,32000] 130 -> 123 us and
-// [256,32000].[32000,1024] 129 -> 107 us; 4096^3 943 -> 769 us, with B stored [N][K] 948 -> 757, A stored [K][M] 925 -> 770, both 946 -> 768.
-// The matrix instructions alone take about 490 us of that (the card holds about 1.75 GHz under them); cutting, adding and writing to LDS is what
-// does not hide behind them. Measured and dropped: all six products in one sum, added every 32 k (735 us, and the loss above),
-// slabs of 32 with two barriers, fetching two slabs ahead (no faster, registers), subtracting with v_dot2_f32_bf16 (slower and not
-// exact).
+// Measured (normal operands, steady load): [256,1024].[1024,32000] 145 -> 116 us, its gradients [1024,256].[256,32000] 130 -> 123 us and
+// [256,32000].[32000,1024] 129 -> 107 us; 4096^3 943 -> 769 us, with B stored [N][K] 948 -> 757, A stored [K][M] 925 -> 770, both 946 -> 768. After
+// idle time both sides are slower: 162 -> 125, 160 -> 148, 157 -> 125, 4096^3 1102 -> 995. What bounds it: the matrix instructions
+// fill 0.39 (second of these) and 0.52 (third) of the cycles, cutting and adding 0.44 and 0.43, and the two hardly overlap. Measured and
+// dropped: all six products in one sum, added every 32 k (735 us at 4096^3, and the loss above), slabs of 32 with two barriers,
+// fetching two slabs ahead (spills: 1260 us), both first slabs of a tile at once (800), an order of instructions within the groups (776), no order
+// between them (776 to 795), subtracting with v_dot2_f32_bf16 (slower and not exact).
 //
 // LDS rows are 32 bytes, two 16-byte granules of eight k. Granule g of row r lies in slot g ^ (bit 2 of r) of the row whose bit 2 is
 // flipped where bit 3 of r is set: eight neighbouring rows touch eight different 16-byte columns of 128 bytes, sixteen touch sixteen of

@@ -393,7 +393,8 @@ def test_sgemm_many_tiles_walked_by_one_workgroup_per_compute_unit(gpu, rng, M, 
     unit walks a list of tiles, the part of the inner extent beyond whole 32-deep slabs is added by a second launch. Padded
     leading dimensions with NaN in every padding (nothing outside the operands may reach a result, tiles that hang over the
     edges of C included), alpha and beta, then beta = 0 over a destination full of NaN; against the product in double
-    precision, every element."""
+    precision, every element. (The largest of these shapes go to the split product; tests/test_gpu_split_product.py has such shapes with
+    that switched off.)"""
     hip = gpu
     A = rng.randn(M, K).astype(np.float32)
     B = rng.randn(K, N).astype(np.float32)

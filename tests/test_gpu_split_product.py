@@ -67,8 +67,8 @@ def test_whole_numbers_are_exact_and_alpha_beta(gpu):
 
 @pytest.mark.parametrize("shape", [(2040, 2040, 2050), (200, 1000, 32000)])
 def test_values_that_three_bf16_do_not_hold(gpu, shape):
-    """Infinities, NaN, values next to the largest float and values whose last bits lie below the smallest bf16: what the fp32
-    instructions make of them."""
+    """Infinities, NaN and values next to the largest float: what the fp32 instructions make of them. Values whose last bits would lie
+    below the smallest bf16: within the fp32 instructions' tolerance as well."""
     M, N, K = shape
     rng = np.random.RandomState(6)
     a, b = rng.randn(M, K).astype(np.float32), rng.randn(K, N).astype(np.float32)
