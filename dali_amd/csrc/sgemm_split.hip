@@ -15,16 +15,18 @@
 // that a single entry below 2^-110, as a softmax gradient has where a logit lies 76 below the largest, loses bits.
 // Infinities, NaN, values from about 2^112 and sums from 2^96 on leave a scaled sum that is not finite: such a tile is redone
 // with the fp32 instructions on the values as they are, whatever they come to. [256,1024].[1024,32000]: one entry in 61 below 2^-110
-// 99 us as without them (246 while the last piece lost bits and such tiles were redone), a NaN in every strip of rows 234
+// 106 us as without them (246 while the last piece lost bits and such tiles were redone), a NaN in every strip of rows 244
 // us, the fp32 kernels 138.
 //
-// A MFMA of this kind cuts off (does not round) what an addend has below about 2^-25 of the largest: small products added to a large sum
-// lose their ends, over a whole inner extent and within one product alike. So the five small products have sums of their
+// A MFMA of this kind takes an accumulator that is smaller than the sum of products added to it down to a multiple of 2^-24 of that sum's
+// power of two (towards minus infinity) before it rounds the result; where the accumulator is the larger one the result is rounded to
+// nearest (probed with single products). Small products summed first lose their ends when hh is added. So the five small products have sums of their
 // own, a 2^-8 of the result, where that does not matter; hh is summed over two slabs (32 values of k) from zero and added to
 // the sums by the vector unit, as are the small ones at the end. Distance from double precision, results of [2048,2048], normal
 // operands (in brackets the fp32 kernels): K = 133 0.58e-7 (2.0e-7), 512 0.86e-7 (4.1e-7), 1999 1.2e-7 (7.9e-7); [1024,1024] over 32000 2.2e-7
 // (2.3e-6). Rows of one product only (a diagonal operand) 2.58e-8 in the root mean square and 9.9e-8 at worst (2.53e-8, 6.0e-8: an
-// fp32 product rounded once), two and more in a row already less than there. With all six in one sum a diagonal operand showed 3.3e-8 and
+// fp32 product rounded once), two and more of like size in a row already less than there; where a few of very different
+// sizes make up a result (exponents spread evenly over e^-20 to e^20, K = 65) 5.3e-8 (5.1e-8). With all six in one sum a diagonal operand showed 3.3e-8 and
 // 15.7e-8; with the two largest of those left out as well, 2.53e-8 and 6.0e-8, but at 131, 144 and 130 us for the three products
 // below, which is the time of the fp32 kernels.
 //
@@ -38,7 +40,8 @@
 // [256,32000].[32000,1024] 129 -> 107 us; 4096^3 943 -> 769 us, with B stored [N][K] 948 -> 757, A stored [K][M] 925 -> 770, both 946 -> 768. After
 // idle time both sides are slower: 162 -> 125, 160 -> 148, 157 -> 125, 4096^3 1102 -> 995. What bounds it: the matrix instructions
 // fill 0.39 (second of these) and 0.52 (third) of the cycles, cutting and adding 0.44 and 0.43, and the two hardly overlap. Measured and
-// dropped: all six products in one sum, added every 32 k (735 us at 4096^3, and the loss above), slabs of 32 with two barriers,
+// dropped: all six products in one sum, added every 32 k (735 us at 4096^3, and the loss above), hh added to the sums by the matrix
+// instruction itself (710, but 1.28e-7 at K = 512 and 4.0e-7 at 32000, further off than the form before), slabs of 32 with two barriers,
 // fetching two slabs ahead (spills: 1260 us), both first slabs of a tile at once (800), an order of instructions within the groups (776), no order
 // between them (776 to 795), subtracting with v_dot2_f32_bf16 (slower and not exact).
 //
