@@ -329,7 +329,8 @@ struct SmallStepArgs {
     float* Cout;      // [B, H]
     float* Hout;      // [B, H]
     int ldx, ldh, ldw, ldu;
-    unsigned int* tickets;  // one per unit block, zero at rest
+    unsigned int* tickets;  // one per unit block, zero at rest, ticket_step words apart
+    int ticket_step;
     float* partials;        // [unit blocks][4 gates][KS][B][64]
 };
 
@@ -405,7 +406,7 @@ __global__ __launch_bounds__(256) void lstm_step_small_kernel(SmallStepArgs a) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
-        const unsigned int ticket = __hip_atomic_fetch_add(a.tickets + ub, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned int ticket = __hip_atomic_fetch_add(a.tickets + ub * a.ticket_step, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         is_last = ticket == (unsigned int)(4 * KS - 1);
     }
     __syncthreads();
@@ -470,7 +471,7 @@ __global__ __launch_bounds__(256) void lstm_step_small_kernel(SmallStepArgs a) {
     };
     if (KS <= 4 && quads > 256) fold(std::integral_constant<int, 2>(), std::integral_constant<int, 4>());
     else fold(std::integral_constant<int, 1>(), std::integral_constant<int, kSmallMaxShares>());
-    if (tid == 0) __hip_atomic_store(a.tickets + ub, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) __hip_atomic_store(a.tickets + ub * a.ticket_step, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 static int* g_status = nullptr;  // pinned host word the kernel raises on a barrier time-out
@@ -654,6 +655,7 @@ extern "C" int dali_hip_lstm_step_small(int batch, int input, int hidden, const 
     a.X = X; a.Hp = Hprev; a.Cp = Cprev; a.W = W; a.U = U; a.bias = bias; a.Cout = Cout; a.Hout = Hout;
     a.ldx = ldx; a.ldh = ldh; a.ldw = ldw; a.ldu = ldu;
     a.tickets = (unsigned int*)workspace();
+    a.ticket_step = counter_step(unit_blocks);
     a.partials = (float*)(workspace() + kWorkspaceCounterBytes);
     const int MT = (batch + 15) / 16, grid = unit_blocks * 4 * KS;
     const size_t lds_bytes = (size_t)4 * 4 * MT * 256 * sizeof(float);

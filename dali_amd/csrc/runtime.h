@@ -17,6 +17,13 @@ constexpr int kWorkspaceCounters = 16384;
 constexpr size_t kWorkspaceCounterBytes = (size_t)kWorkspaceCounters * 4;
 constexpr size_t kWorkspacePartialBytes = (size_t)32 << 20;
 constexpr size_t kWorkspaceBytes = kWorkspaceCounterBytes + kWorkspacePartialBytes;
+// Words between n of the counters that are drawn from at the same time: memory takes an arrival every 12 ns or so at one cache line,
+// whichever word it goes to, so they lie 256 bytes apart as far as there is room.
+inline int counter_step(long n) {
+    int step = 64;
+    while (step > 1 && step * n > kWorkspaceCounters) step /= 2;
+    return step;
+}
 
 int fail(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 int fail_str(const std::string& s);

@@ -73,7 +73,8 @@ struct GemmArgs {
     float alpha, beta;
     // split-K: gridDim.z workgroups share one tile of C, each walking a contiguous share of the
     // slabs; partial tiles and the per-tile ticket counters live in the library workspace
-    unsigned int* counters;
+    unsigned int* counters;  // counter_step words apart
+    int counter_step;
     float* partials;
     // fused LSTM gate epilogue (GATES kernels): C is not written; the tile's pre-activations go through the
     // gate arithmetic with bias[4H], c_prev[M, H] and leave as c_out[M, H], h_out[M, H]
@@ -670,7 +671,7 @@ __global__ __launch_bounds__(256 * KW, (BM == 128 && !EDGE && KW == 1) ? 2 : 1) 
         __shared__ int is_last;
         __syncthreads();
         if (tid == 0) {
-            unsigned int ticket = __hip_atomic_fetch_add(g.counters + tile_id, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            unsigned int ticket = __hip_atomic_fetch_add(g.counters + tile_id * g.counter_step, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             is_last = ticket == gridDim.z - 1;
         }
         __syncthreads();
@@ -732,7 +733,7 @@ __global__ __launch_bounds__(256 * KW, (BM == 128 && !EDGE && KW == 1) ? 2 : 1) 
                 }
             }
         }
-    if (split && tid == 0) __hip_atomic_store(g.counters + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (split && tid == 0) __hip_atomic_store(g.counters + tile_id * g.counter_step, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 template <int BM, int BN, int BK, int DEPTH, int KW = 1, bool MIDB = false>
@@ -747,6 +748,7 @@ static int launch_tile(GemmArgs g, bool ta, bool tb, bool vec, int split_k, bool
     if (split_k > 1 && (tiles > (size_t)kWorkspaceCounters || tiles * split_k * BM * BN * sizeof(float) > kWorkspacePartialBytes)) split_k = 1;
     grid.z = split_k;
     g.counters = (unsigned int*)workspace();
+    g.counter_step = counter_step((long)tiles);
     g.partials = (float*)(workspace() + kWorkspaceCounterBytes);
     dim3 block(256 * KW);
     hipStream_t st = stream();

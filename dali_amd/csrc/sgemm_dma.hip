@@ -420,7 +420,8 @@ struct StreamArgs {
     int ldc;
     float alpha, beta;
     int tiles_m, tiles_n, Z;
-    unsigned int* counters;  // one ticket counter per tile (zero at rest)
+    unsigned int* counters;  // one ticket counter per tile (zero at rest), counter_step words apart
+    int counter_step;
     float* partials;         // [tile][share][4096]
     // gate epilogue (GATES): C is not written; a tile's columns are the four gates of sixteen hidden units
     const float* bias;
@@ -655,7 +656,7 @@ __global__ __launch_bounds__(512, 1) void sgemm_dma_stream_kernel(StreamArgs g) 
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             __syncthreads();
             if (tid == 0) {
-                const unsigned int ticket = __hip_atomic_fetch_add(g.counters + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const unsigned int ticket = __hip_atomic_fetch_add(g.counters + tile * g.counter_step, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 is_last = ticket == (unsigned int)Z - 1;
             }
             __syncthreads();
@@ -677,7 +678,7 @@ __global__ __launch_bounds__(512, 1) void sgemm_dma_stream_kernel(StreamArgs g) 
                             for (int v = 0; v < 8; ++v) sum[v] += t[u][v];
                         }
                 }
-                if (tid == 0) __hip_atomic_store(g.counters + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (tid == 0) __hip_atomic_store(g.counters + tile * g.counter_step, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
         if (GATES) {
@@ -878,6 +879,7 @@ int sgemm_dma_stream(bool ta, bool tb, int M, int N, int nseg, const int* K, con
     g.h_out = h_out;
     g.H = H;
     g.counters = (unsigned int*)workspace();
+    g.counter_step = counter_step(tiles);
     g.partials = (float*)(workspace() + kWorkspaceCounterBytes);
     const long items = tiles * Z;
     // every workgroup has a compute unit to itself (its LDS); a whole number of workgroups per die keeps the bands of tiles

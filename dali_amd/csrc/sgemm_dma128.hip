@@ -53,7 +53,8 @@ struct Args128 {
     // workgroups) are either worked whole by the first `rem` workgroups (shares = 0) or cut along the inner extent into equal
     // shares, one per workgroup (boundaries within `min_frag` slabs of a tile's edge move to the edge).
     int rounds, rem, shares, min_frag;  // shares: workgroups that take a share of the left-over tiles (0: those tiles go whole)
-    unsigned int* counters;  // one ticket counter per left-over tile (zero at rest)
+    unsigned int* counters;  // one ticket counter per left-over tile (zero at rest), counter_step words apart
+    int counter_step;
     float* partials;         // [2 * workgroups][128 * 128]: a workgroup's share that starts inside a tile, then the one that ends inside one
 };
 
@@ -357,7 +358,7 @@ __global__ __launch_bounds__(512, 1) void sgemm_dma128_kernel(Args128 g) {
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             __syncthreads();
             if (tid == 0) {
-                const unsigned int ticket = __hip_atomic_fetch_add(g.counters + t, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const unsigned int ticket = __hip_atomic_fetch_add(g.counters + t * g.counter_step, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 is_last = ticket == (unsigned int)sharers - 1;
             }
             __syncthreads();
@@ -395,7 +396,7 @@ __global__ __launch_bounds__(512, 1) void sgemm_dma128_kernel(Args128 g) {
                 for (int i = 0; i < RB; ++i)
 #pragma unroll
                     for (int j = 0; j < 2; ++j) acc[i][j] = sum[i][j];
-                if (tid == 0) __hip_atomic_store(g.counters + t, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (tid == 0) __hip_atomic_store(g.counters + t * g.counter_step, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
         int mt, nt;
@@ -615,6 +616,7 @@ int sgemm_dma128(bool ta, bool tb, int M, int N, int K, const float* A, int lda,
     g.shares = share ? (4 * rest < workgroups ? 4 * rest : workgroups) : 0;
     g.min_frag = 2;
     g.counters = (unsigned int*)workspace();
+    g.counter_step = counter_step(rest > 0 ? rest : 1);
     g.partials = (float*)(workspace() + kWorkspaceCounterBytes);
     if (low) return kt ? launch128<false, false, 64, false, true>(g, workgroups) : launch128<false, false, 64, false>(g, workgroups);
     if (kt) {

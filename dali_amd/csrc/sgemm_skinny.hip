@@ -35,7 +35,8 @@ struct SkinnyArgs {
     float* C;
     int lda, ldb, ldc;
     float alpha, beta;
-    unsigned int* tickets;  // one per column block, zero at rest
+    unsigned int* tickets;  // one per column block, zero at rest, ticket_step words apart
+    int ticket_step;
     float* partials;        // [column blocks][KS][M][64]
 };
 
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(256, 2) void sgemm_skinny_kernel(SkinnyArgs a) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
-        const unsigned int ticket = __hip_atomic_fetch_add(a.tickets + cb, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned int ticket = __hip_atomic_fetch_add(a.tickets + cb * a.ticket_step, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         is_last = ticket == (unsigned int)(KS - 1);
     }
     __syncthreads();
@@ -154,7 +155,7 @@ __global__ __launch_bounds__(256, 2) void sgemm_skinny_kernel(SkinnyArgs a) {
                 *p = a.beta == 0.0f ? s : s + a.beta * *p;
             }
     }
-    if (tid == 0) __hip_atomic_store(a.tickets + cb, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) __hip_atomic_store(a.tickets + cb * a.ticket_step, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---------------------------------------------------------------------------------------------- short inner extent
@@ -268,6 +269,7 @@ int sgemm_skinny(bool tb, int M, int N, int K, float alpha, const float* A, int 
     a.lda = lda; a.ldb = ldb; a.ldc = ldc;
     a.alpha = alpha; a.beta = beta;
     a.tickets = (unsigned int*)workspace();
+    a.ticket_step = counter_step(blocks);
     a.partials = (float*)(workspace() + kWorkspaceCounterBytes);
     const int MT = (M + 15) / 16;
     const size_t lds_bytes = (size_t)4 * 4 * MT * 256 * sizeof(float);

@@ -349,6 +349,35 @@ DI void dali_publish(dali_ms* p, dali_ms v) {
 DI dali_ms dali_observe(const dali_ms* p) {
     return __builtin_bit_cast(dali_ms, __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
+// The same for N neighbouring values of a lane, `bytes` into the workspace's partial results (`base`, the same for the whole wave), as 16-byte
+// accesses at device scope: the coherence point takes a wave's access per cache line it touches, whatever the access brings, so
+// values moved one by one cost four times the requests.
+constexpr int kDeviceScope = 16;  // cache policy of a buffer access
+typedef unsigned int dali_u4 __attribute__((ext_vector_type(4)));
+template <typename T, int N> DI void dali_publish_vec(void* base, unsigned int bytes, const T* v) {
+    if constexpr (sizeof(T) * N % 16 == 0) {
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(base, 0, 32 << 20, 0x00027000);
+        struct alignas(16) words { dali_u4 w[sizeof(T) * N / 16]; } u;
+        __builtin_memcpy(&u, v, sizeof(u));
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof(T) * N / 16); ++i) __builtin_amdgcn_raw_buffer_store_b128(u.w[i], rsrc, bytes + 16 * i, 0, kDeviceScope);
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j) dali_publish(reinterpret_cast<T*>(static_cast<char*>(base) + bytes) + j, v[j]);
+    }
+}
+template <typename T, int N> DI void dali_observe_vec(void* base, unsigned int bytes, T* v) {
+    if constexpr (sizeof(T) * N % 16 == 0) {
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(base, 0, 32 << 20, 0x00027000);
+        struct alignas(16) words { dali_u4 w[sizeof(T) * N / 16]; } u;
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof(T) * N / 16); ++i) u.w[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, bytes + 16 * i, 0, kDeviceScope);
+        __builtin_memcpy(v, &u, sizeof(u));
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j) v[j] = dali_observe(reinterpret_cast<const T*>(static_cast<char*>(base) + bytes) + j);
+    }
+}
 // Waits until this thread's earlier stores are acknowledged by memory; also a compiler barrier for memory operations.
 DI void dali_stores_acknowledged() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory"); }
 // Waits until this thread's earlier stores are acknowledged by memory, then draws a ticket. The wait is written as an asm
@@ -361,19 +390,28 @@ DI unsigned int dali_take_ticket(unsigned int* counter) {
     return ticket;
 }
 
-// Whether workgroup b is the last of n to arrive. One counter takes an arrival every 12 ns or so, whoever asks: tens of
-// thousands of workgroups of a short kernel would queue for it (65536 rows of 513 in one launch: 200 us, of which 130 us
-// waiting for tickets). From 1024 workgroups on they arrive in 64 groups with a counter each, counters[1 + group], and the
+// Words between n ticket counters that are drawn from at the same time. Memory takes an arrival every 12 ns or so at one cache line,
+// whichever word it goes to, so the counters lie on lines of their own (256 bytes apart) as far as the workspace's 16384 words allow.
+DI unsigned int dali_counter_step(unsigned int n) { return n <= 256 ? 64u : (n > 8192 ? 1u : 16384u >> (32 - __builtin_clz(n - 1))); }
+
+// Whether workgroup b is the last of n to arrive. Arrivals at one counter queue: tens of thousands of workgroups of a short
+// kernel would wait for their tickets longer than they work (65536 rows of 513 in one launch: 200 us, of which 130 us
+// tickets). From GROUPED workgroups on they arrive in 16 groups, from 1024 on in 64, with a counter each behind counters[0], and the
 // last of a group, which sets its counter back to zero, draws from counters[0] for the group. Every arrival has had its
 // earlier stores acknowledged, so what all of them published is in memory when the last one is told so. counters[0] is left
-// at n (or 64) for the caller to set back.
+// at n (or the number of groups) for the caller to set back. Cross-entropy with its mean, us, the groups' counters side by side and
+// on lines of their own: [4096,1000] 26.3 -> 9.9, [16000,1000] 88.7 -> 31.2; one counter, 16 groups: [256,1000] 6.9 -> 5.3, [1000,1000]
+// 15.7 -> 6.3, the maximum of [4096,1024] 9.1 -> 4.8. (Workgroups that work for ten microseconds and more arrive spread out, and what a
+// group costs is the second round trip: rows of 32000 keep one counter up to 1024, [512,32000] 21.1, in groups 22.1.)
+template <unsigned int GROUPED = 128>
 DI bool dali_last_arrival(unsigned int* counters, unsigned int b, unsigned int n) {
-    constexpr unsigned int kGroups = 64;
-    if (n < 1024) return dali_take_ticket(&counters[0]) == n - 1;
-    const unsigned int group = b % kGroups, members = (n - group + kGroups - 1) / kGroups;
-    if (dali_take_ticket(&counters[1 + group]) != members - 1) return false;
-    dali_publish(&counters[1 + group], 0u);
-    return dali_take_ticket(&counters[0]) == kGroups - 1;
+    if (n < GROUPED) return dali_take_ticket(&counters[0]) == n - 1;
+    const unsigned int groups = n < 1024 ? 16 : 64;
+    const unsigned int group = b % groups, members = (n - group + groups - 1) / groups;
+    unsigned int* own = counters + (1 + group) * 64;
+    if (dali_take_ticket(own) != members - 1) return false;
+    dali_publish(own, 0u);
+    return dali_take_ticket(&counters[0]) == groups - 1;
 }
 
 // --------------------------------------------------------- cross-lane helpers

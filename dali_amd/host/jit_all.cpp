@@ -73,14 +73,14 @@ static std::string gen_all_kernel(const Program& P, int red_id, int root_id, int
     // atomic stores (written through to the device coherence point, never left dirty in one
     // XCD's L2), s_waitcnt 0 holds the ticket back until those stores are acknowledged, and the
     // last block reads them with agent-scope atomic loads (which do not hit stale lines).
-    ss << "  if (threadIdx.x == 0) {\n    dali_publish(&partials[blockIdx.x].v, acc); dali_publish(&partials[blockIdx.x].i, acci);\n"
-          "    is_last = dali_take_ticket(&counters[0]) == gridDim.x - 1;\n  }\n  __syncthreads();\n";
+    ss << "  if (threadIdx.x == 0) {\n    dali_publish(&partials[blockIdx.x].v, acc);" << (is_arg ? " dali_publish(&partials[blockIdx.x].i, acci);" : "") << "\n"
+          "    is_last = dali_last_arrival(counters, blockIdx.x, gridDim.x);\n  }\n  __syncthreads();\n";
     ss << "  if (!is_last) return;\n";
     ss << "  acc = " << red.name << "::init<" << t << ">(); acci = 0;\n";
     ss << "  // fixed combination order: thread k folds partials k, k+BT, ... (all loads issued first), then the block folds in wave order\n";
-    ss << "  {\n    constexpr int TAIL = " << TAIL << ";\n    " << t << " pv[TAIL]; int pi[TAIL];\n";
+    ss << "  {\n    constexpr int TAIL = " << TAIL << ";\n    " << t << " pv[TAIL];" << (is_arg ? " int pi[TAIL];" : "") << "\n";
     ss << "    _Pragma(\"unroll\") for (int k = 0; k < TAIL; ++k) {\n      const unsigned int b = threadIdx.x + k * BT;\n"
-          "      if (b < gridDim.x) { pv[k] = dali_observe(&partials[b].v); pi[k] = dali_observe(&partials[b].i); }\n    }\n";
+          "      if (b < gridDim.x) { pv[k] = dali_observe(&partials[b].v);" << (is_arg ? " pi[k] = dali_observe(&partials[b].i);" : "") << " }\n    }\n";
     ss << "    _Pragma(\"unroll\") for (int k = 0; k < TAIL; ++k) {\n      const unsigned int b = threadIdx.x + k * BT;\n      if (b < gridDim.x) {\n";
     if (!is_arg)
         ss << "        acc = " << red.name << "::step<" << t << ">(acc, pv[k]);\n";

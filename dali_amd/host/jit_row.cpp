@@ -330,7 +330,7 @@ static std::string gen_row_kernel(const RowPlan& rpn, const IvLayout& L, const s
             const std::string t = ctype(P.nodes[P.nodes[totals[k]->total_red].args[0]].dtype);
             ss << "    dali_publish((" << t << "*)(slots + ((size_t)" << k << " * gridDim.x + blockIdx.x) * 8), tot" << k << ");\n";
         }
-        ss << "    is_last = dali_last_arrival(counters, blockIdx.x, gridDim.x);\n  }\n";
+        ss << "    is_last = dali_last_arrival<" << (rpn.dom.C >= 16384 ? 1024 : 128) << ">(counters, blockIdx.x, gridDim.x);\n  }\n";
     };
     auto emit_totals_fold = [&]() {
         ss << "  __syncthreads();\n  if (!is_last) return;\n";
@@ -865,7 +865,7 @@ bool try_row(const std::vector<DestSpec>& specs, const Domain& dom, const std::v
         // one 8-byte slot per workgroup and total in the workspace's 32 MiB of partial results
         const int64_t blocks = (dom.R + rp.RPB - 1) / rp.RPB;
         if (blocks * (int64_t)n_totals * 8 > ((int64_t)32 << 20) || blocks > 2147483647LL) return false;
-        params << ",T" << n_totals;
+        params << ",T" << n_totals << (dom.C >= 16384 ? "L" : "");
     }
     static std::unordered_map<uint64_t, std::shared_ptr<KernelSpec>> specs_cache;
     std::string sig = signature(P, rpn.outputs);
