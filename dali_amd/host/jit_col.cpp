@@ -203,14 +203,26 @@ static std::string gen_col_kernel(const Program& P, int red_id, int dest_array, 
             else
             ss << be.stmts.str() << "          acc[j] = " << feed << "acc[j], " << v << ");\n        }\n      }\n";
     }
+    // (few y-blocks leave a row group up to UNR - 1 rows behind its chunks: four in flight at a time; long arithmetic is not copied four times)
+    const int RST = contains_expensive(P, red.args[0]) ? 1 : 4;
     if (IL == 2)
-        ss << "    }\n    for (long x = n_chunks * (UNR * NWAVE) + (long)blockIdx.y * NWAVE + wave; x < x_end; x += (long)gridDim.y * NWAVE) {\n";
+        ss << "    }\n    const long rest_step = (long)gridDim.y * NWAVE;\n    constexpr int RST = " << RST << ";\n    for (long r = n_chunks * (UNR * NWAVE) + (long)blockIdx.y * NWAVE + wave; r < x_end; r += RST * rest_step) {\n";
     else
         ss << "    }\n    for (; x < x_end; x += XS) {\n";
     for (int i : full_leaves) {
         std::string ty = ctype(P.arrays[i].buf->dtype);
+        if (IL == 2) {
+            ss << "      " << ty << " x" << i << "s[RST][VEC];\n";
+            ss << "      _Pragma(\"unroll\") for (int u = 0; u < RST; ++u) if (r + u * rest_step < x_end) { dali_vec<" << ty << ", VEC> tmp = " << ld << ty << ", VEC>(q" << i
+               << " + (r + u * rest_step) * ld" << i << "); _Pragma(\"unroll\") for (int j = 0; j < VEC; ++j) x" << i << "s[u][j] = tmp.v[j]; }\n";
+            continue;
+        }
         ss << "      " << ty << " x" << i << "[VEC];\n";
         ss << "      { dali_vec<" << ty << ", VEC> tmp = " << ld << ty << ", VEC>(q" << i << " + x * ld" << i << "); _Pragma(\"unroll\") for (int j = 0; j < VEC; ++j) x" << i << "[j] = tmp.v[j]; }\n";
+    }
+    if (IL == 2) {
+        ss << "      _Pragma(\"unroll\") for (int u = 0; u < RST; ++u) if (r + u * rest_step < x_end) {\n      const long x = r + u * rest_step; (void)x;\n";
+        for (int i : full_leaves) ss << "      const " << ctype(P.arrays[i].buf->dtype) << "* x" << i << " = x" << i << "s[u];\n";
     }
     ss << "      _Pragma(\"unroll\") for (int j = 0; j < VEC; ++j) {\n        const int col = 0; (void)col;\n";
     for (int i : kept_vectors) ss << "        const " << ctype(P.arrays[i].buf->dtype) << " rl" << i << " = rl" << i << "v[j];\n";
@@ -222,22 +234,24 @@ static std::string gen_col_kernel(const Program& P, int red_id, int dest_array, 
         else
             ss << be.stmts.str() << "        acc[j] = " << feed << "acc[j], " << v << ");\n      }\n";
     }
+    if (IL == 2) ss << "      }\n";
     ss << "    }\n  }\n";
-    // fold the row groups of the block in group order
+    // fold the row groups of the block in group order: a thread per column of the strip, then back to the lanes of the first group
     ss << "  __shared__ " << t << " sm[NWAVE][TPP * VEC];\n  __shared__ int is_last;\n";
     if (ARG) ss << "  __shared__ int smi[NWAVE][TPP * VEC];\n";
     auto emit_group_fold = [&](const std::string& ind) {
         ss << ind << "if (NWAVE > 1) {\n" << ind << "  _Pragma(\"unroll\") for (int j = 0; j < VEC; ++j) { sm[wave][lane * VEC + j] = acc[j];" << (ARG ? " smi[wave][lane * VEC + j] = acci[j];" : "")
            << " }\n" << ind << "  __syncthreads();\n";
-        ss << ind << "  if (wave == 0) {\n" << ind << "    _Pragma(\"unroll\") for (int j = 0; j < VEC; ++j) {\n" << ind << "      " << t << " r = sm[0][lane * VEC + j];\n";
+        ss << ind << "  if (threadIdx.x < TPP * VEC) {\n" << ind << "    " << t << " r = sm[0][threadIdx.x];\n";
         if (ARG) {
-            ss << ind << "      int ri = smi[0][lane * VEC + j];\n";
-            ss << ind << "      _Pragma(\"unroll\") for (int w = 1; w < NWAVE; ++w) { const " << t << " ov = sm[w][lane * VEC + j]; const int oi = smi[w][lane * VEC + j]; " << take("r", "ri", "ov", "oi") << " }\n";
-            ss << ind << "      acc[j] = r; acci[j] = ri;\n";
+            ss << ind << "    int ri = smi[0][threadIdx.x];\n";
+            ss << ind << "    _Pragma(\"unroll\") for (int w = 1; w < NWAVE; ++w) { const " << t << " ov = sm[w][threadIdx.x]; const int oi = smi[w][threadIdx.x]; " << take("r", "ri", "ov", "oi") << " }\n";
+            ss << ind << "    sm[0][threadIdx.x] = r; smi[0][threadIdx.x] = ri;\n";
         } else {
-            ss << ind << "      _Pragma(\"unroll\") for (int w = 1; w < NWAVE; ++w) r = " << red.name << "::step<" << t << ">(r, sm[w][lane * VEC + j]);\n" << ind << "      acc[j] = r;\n";
+            ss << ind << "    _Pragma(\"unroll\") for (int w = 1; w < NWAVE; ++w) r = " << red.name << "::step<" << t << ">(r, sm[w][threadIdx.x]);\n" << ind << "    sm[0][threadIdx.x] = r;\n";
         }
-        ss << ind << "    }\n" << ind << "  }\n" << ind << "}\n";
+        ss << ind << "  }\n" << ind << "  __syncthreads();\n" << ind << "  if (wave == 0) {\n" << ind << "    _Pragma(\"unroll\") for (int j = 0; j < VEC; ++j) { acc[j] = sm[0][lane * VEC + j];"
+           << (ARG ? " acci[j] = smi[0][lane * VEC + j];" : "") << " }\n" << ind << "  }\n" << ind << "}\n";
     };
     emit_group_fold("  ");
     auto emit_store = [&](const std::string& indent) {
@@ -252,17 +266,21 @@ static std::string gen_col_kernel(const Program& P, int red_id, int dest_array, 
     ss << "  if (gridDim.y == 1) {\n    if (wave == 0 && k_ok) {\n";
     emit_store("      ");
     ss << "    }\n    return;\n  }\n";
-    ss << "  unsigned int* counters = (unsigned int*)A.ws;\n";
-    ss << "  " << t << "* partials = (" << t << "*)((char*)A.ws + " << 16384 * 4 << ");\n";
-    ss << "  const long KP = (long)gridDim.x * TPP * VEC;  // padded kept extent of one row of partials\n";
-    ss << "  const long pcol = ((long)blockIdx.x * TPP + lane) * VEC;\n";
+    // one counter a strip; a few strips with many workgroups each have groups of them (up to 16 behind the strip's own)
+    ss << "  const bool grouped = gridDim.x <= 15;\n";
+    ss << "  unsigned int* counters = (unsigned int*)A.ws + (grouped ? blockIdx.x * (17u * 64u) : blockIdx.x * dali_counter_step(gridDim.x));\n";
+    ss << "  char* partials = (char*)A.ws + " << 16384 * 4 << ";\n";
+    ss << "  const unsigned int KP = gridDim.x * TPP * VEC;  // padded kept extent of one row of partials\n";
+    ss << "  const unsigned int pcol = (blockIdx.x * TPP + lane) * VEC;\n";
     // same fence-free hand-off as the full reduction: agent-scope atomic stores, wait for their
     // acknowledgement, then the ticket; the last block of the strip observes with agent-scope loads
-    if (ARG) ss << "  int* pidx = (int*)(partials + (long)gridDim.y * KP);  // the indices follow the values\n";
-    ss << "  if (wave == 0) {\n    _Pragma(\"unroll\") for (int j = 0; j < VEC; ++j) { dali_publish(partials + (long)blockIdx.y * KP + pcol + j, acc[j]);"
-       << (ARG ? " dali_publish(pidx + (long)blockIdx.y * KP + pcol + j, acci[j]);" : "") << " }\n"
-          "    dali_stores_acknowledged();\n  }\n  __syncthreads();\n";
-    ss << "  if (threadIdx.x == 0) is_last = dali_take_ticket(&counters[blockIdx.x]) == gridDim.y - 1;\n  __syncthreads();\n";
+    if (ARG) ss << "  const unsigned int indices = gridDim.y * KP * (unsigned int)sizeof(" << t << ");  // the indices follow the values\n";
+    auto value_at = [&](const std::string& y) { return "(" + y + " * KP + pcol) * (unsigned int)sizeof(" + t + ")"; };
+    auto index_at = [&](const std::string& y) { return "indices + (" + y + " * KP + pcol) * 4u"; };
+    ss << "  if (wave == 0) {\n    dali_publish_vec<" << t << ", VEC>(partials, " << value_at("blockIdx.y") << ", acc);\n";
+    if (ARG) ss << "    dali_publish_vec<int, VEC>(partials, " << index_at("blockIdx.y") << ", acci);\n";
+    ss << "    dali_stores_acknowledged();\n  }\n  __syncthreads();\n";
+    ss << "  if (threadIdx.x == 0) is_last = grouped ? dali_last_arrival(counters, blockIdx.y, gridDim.y) : dali_take_ticket(counters) == gridDim.y - 1;\n  __syncthreads();\n";
     ss << "  if (!is_last) return;\n";
     // every row group of the last block folds a contiguous share of the partial rows in y order (TAIL of them in
     // flight at a time); the groups are then joined in group order through LDS
@@ -273,8 +291,9 @@ static std::string gen_col_kernel(const Program& P, int red_id, int dest_array, 
     ss << "  for (unsigned int y0 = y_begin; y0 < y_end; y0 += TAIL) {\n    dali_vec<" << t << ", VEC> pv[TAIL];\n";
     if (ARG) ss << "    dali_vec<int, VEC> pi[TAIL];\n";
     ss << "    _Pragma(\"unroll\") for (int k = 0; k < TAIL; ++k) if (y0 + k < y_end) {\n"
-          "      _Pragma(\"unroll\") for (int j = 0; j < VEC; ++j) { pv[k].v[j] = dali_observe(partials + (long)(y0 + k) * KP + pcol + j);"
-       << (ARG ? " pi[k].v[j] = dali_observe(pidx + (long)(y0 + k) * KP + pcol + j);" : "") << " }\n    }\n";
+          "      dali_observe_vec<" << t << ", VEC>(partials, " << value_at("(y0 + k)") << ", pv[k].v);\n";
+    if (ARG) ss << "      dali_observe_vec<int, VEC>(partials, " << index_at("(y0 + k)") << ", pi[k].v);\n";
+    ss << "    }\n";
     if (ARG)
         // the y-blocks hold interleaved chunks of rows: equal values are settled by the index itself
         ss << "    _Pragma(\"unroll\") for (int k = 0; k < TAIL; ++k) if (y0 + k < y_end) {\n      _Pragma(\"unroll\") for (int j = 0; j < VEC; ++j) { "
@@ -285,7 +304,7 @@ static std::string gen_col_kernel(const Program& P, int red_id, int dest_array, 
     emit_group_fold("  ");
     ss << "  if (wave == 0 && k_ok) {\n";
     emit_store("    ");
-    ss << "  }\n  if (threadIdx.x == 0) dali_publish(&counters[blockIdx.x], 0u);\n}\n";
+    ss << "  }\n  if (threadIdx.x == 0) dali_publish(counters, 0u);\n}\n";
     return ss.str();
 }
 
@@ -385,7 +404,7 @@ bool try_col(const DestSpec& spec) {
     int VEC = vec ? 4 : 1;
     const bool UNALIGNED = VEC > 1 && !aligned, SHIFT = VEC > 1 && K % VEC != 0;
     static const int IL = env_int("DALI_HIP_COL_INTERLEAVE", 2);
-    static const int rg_env = env_int("DALI_HIP_COL_RG", 0), tail_env = env_int("DALI_HIP_COL_TAIL", 16);
+    static const int rg_env = env_int("DALI_HIP_COL_RG", 0), tail_env = env_int("DALI_HIP_COL_TAIL", 0);
     static const int unr_env = env_int("DALI_HIP_COL_UNR", 8), rows_env = env_int("DALI_HIP_COL_ROWS", 0);
     static const int blocks_env = env_int("DALI_HIP_COL_BLOCKS", 0);
     // One 256-thread workgroup per CU keeps eight loads per lane in flight and is best for a bare reduction; with
@@ -395,12 +414,19 @@ bool try_col(const DestSpec& spec) {
     const bool streaming = K * X * (int64_t)size_of_dtype(arg.dtype()) >= ((int64_t)64 << 20);
     const int max_blocks = blocks_env > 0 ? blocks_env : (streaming && (pair || contains_expensive(P, P.nodes[red_id].args[0])) ? 512 : 256);
     const int UNR = unr_env;
-    // four row groups of one wave each: a wave reads 1 KiB pieces of memory rows, a block owns a 256-column strip.
-    // Narrow strips and few y-blocks measured best (8192x8192: 53 us with 1024-column strips x 32 y-blocks,
-    // 41 us with 256-column strips x 8 y-blocks).
-    int RG = 4;
+    // Row groups of a workgroup, which owns a strip of 1024 / RG columns. Large matrices of 4-byte values: four of one wave each, a
+    // wave reads 1 KiB pieces of memory rows (8192x8192: 53 us with 1024-column strips x 32 y-blocks, 40 us with 256-column
+    // strips x 8 y-blocks). Smaller ones and 8-byte values (whose 128 columns are 1 KiB again): eight, half as many partial rows to a strip and
+    // twice as many workgroups that fold them ([65536,64] 8.9 -> 6.5 us, [4096,1024] 5.4 -> 4.7, in double precision 12.7 -> 6.1,
+    // [3001,2047] 12.0 -> 9.7, [8192,8192] 92 -> 87). Where a strip can be left to one workgroup, which then meets no others, as
+    // many as its rows keep busy ([100,100] 4.0 -> 2.7, [256,32000] 5.1 -> 3.7, [64,65536] 2.7 with four, 2.9 with sixteen; sixteen with others to meet is
+    // slower: [3001,2047] 6.9 -> 8.2).
+    int RG = streaming && size_of_dtype(arg.dtype()) == 4 ? 4 : 8;
+    if (!streaming && (X <= 256 || (K >= 64 * max_blocks && X <= 1024))) RG = X > 64 ? 16 : (X <= 8 * 4 || K >= 64 * max_blocks ? 4 : 8);
     if (rg_env > 0) RG = rg_env;
-    const int TAIL = tail_env;
+    // partial rows in flight in the fold (sixteen also leave the compiler the registers that exponentials in double precision want in
+    // the main loop: sum(exp(x)) of [8192,8192] 110 us with eight, 97 with sixteen)
+    const int TAIL = tail_env > 0 ? tail_env : (size_of_dtype(arg.dtype()) == 8 && contains_expensive(P, P.nodes[red_id].args[0]) ? 16 : 8);
     std::vector<Output> outs(1);
     outs[0].root = red_id;
     outs[0].array = dest_array;
@@ -429,7 +455,7 @@ bool try_col(const DestSpec& spec) {
         Kp->plan.work_count = 1;
         Kp->plan.work_per_block = (256 / RG) * VEC;
         Kp->plan.work2_begin = L.shape_pos[0] + 1;
-        Kp->plan.work2_per_block = rows_env > 0 ? rows_env : UNR * RG;  // fewest reduced rows per y-block
+        Kp->plan.work2_per_block = rows_env > 0 ? rows_env : (RG == 16 ? 256 : UNR * RG);  // fewest reduced rows per y-block
         Kp->plan.max_blocks2 = maxy_env;
         Kp->plan.max_blocks = max_blocks;  // the y split fills what the column strips leave
         Kp->plan.ws_elsize = pair ? 8 : size_of_dtype(arg.dtype()) + (is_arg ? 4 : 0);  // a partial is a value, plus its index
