@@ -669,8 +669,9 @@ void run_specs_planned(std::vector<DestSpec> specs) {
                     Domain dom = domain_of(first.expression()->args[0].shape());
                     // (tens of thousands of short rows: a workgroup would live as long as its ticket takes to come back, two memory
                     // round trips for a few microseconds of work, and a second small launch over the per-row values is cheaper:
-                    // cross-entropy on [65536,513] 93 -> 51 us, on [100000,1000] 158 -> 142 us)
-                    const bool many_short_rows = dom.C < 2048 && dom.R >= 16384;
+                    // cross-entropy on [65536,513] 93 -> 51 us, on [100000,1000] 158 -> 142 us; with a workgroup to a row already from 8192 on, [8192,1000]
+                    // 16.8 -> 13.4 us)
+                    const bool many_short_rows = dom.C < 2048 && dom.R >= (dom.C >= 640 ? 8192 : 16384);
                     if (!many_short_rows && try_row(plain, dom, &totals)) return;
                 }
             }

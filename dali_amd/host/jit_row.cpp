@@ -585,6 +585,34 @@ static bool peel_ok(const Program& P, const Domain& dom) {
     return off >= 0;
 }
 
+// Threads per row for kernels of two reduction phases and more that write rows of up to 64 vectors (a softmax, a cross-entropy); `whole`: a thread per
+// vector, rounded up to a power of two. Such kernels are bound by instructions, not by memory: a wave whose rows leave lanes idle
+// ([51200,160]: 40 vectors on 64 lanes) issues as many as a full one, and what is done once per row and wave (the folds, the loss) is
+// done for one to four rows at a time. With fewer threads a wave takes more rows and a thread several vectors of its own, at the price of
+// loads and stores of shorter runs of memory. Measured, us, cross-entropy / softmax, a thread per vector -> this rule:
+//   whole cache lines: a quarter of the threads, 8 at least: a run is a line or more. [51200,160] 19.4 / 11.4 -> 12.7 / 9.1, [51200,96] 12.4 / 6.7 -> 9.5 / 4.7,
+//     [26000,256] 12.4 / 6.8 -> 10.3 / 5.6, [250000,160] 98 / 67 -> 58 / 50, [625000,64] 73 / 50 -> 64 / 49
+//   others: half of them. [51200,97] 14.0 / 8.3 -> 11.7 / 6.9, [20000,150] 12.3 / 6.9 -> 10.0 / 5.5, [200000,200] 85 / 55 -> 59 / 53
+//   others of 64 MiB and more, with runs below 512 bytes: only with much arithmetic per element. [400000,100] 86 -> 67 (cross-entropy), but softmax 56 -> 59
+//   fewer than 16 elements without vectors: one thread up to 8 ([8000000,5] 229 / 167 -> 86 / 57), four beyond ([4000000,10] 222 / 169 -> 102 / 74)
+// (Fewer rows than fill the chip with a thread per vector keep that: nothing is gained below 65536 threads.)
+static int short_row_threads(const RowPlan& rpn, int64_t CH, int whole, int n_full, bool big) {
+    bool lines = true;  // rows start at cache lines
+    for (const ArrayArg& a : rpn.P.arrays) {
+        if (a.cls != Cls::FULL || a.gather_source) continue;
+        if (size_of_dtype(a.buf->dtype) != 4) return whole;
+        lines = lines && a.row_stride % 32 == 0 && a.buf->offset % 32 == 0;
+    }
+    int operations = 0;  // per element of a row
+    for (const PNode& n : rpn.P.nodes) operations += n.cls_set && n.cls == Cls::FULL && (n.kind == Kind::ELEMENTWISE || n.kind == Kind::ONE_HOT);
+    int threads = whole;
+    if (rpn.rp.VEC == 1) threads = CH <= 8 ? 1 : CH < 16 ? 4 : whole;
+    else if (lines && rpn.dom.C % 32 == 0) threads = std::min(whole, std::max(8, whole / 4));
+    else if (!big || whole >= 64 || operations >= 5) threads = std::min(whole, std::max(8, whole / 2));
+    // (a thread keeps its values of every operand in registers)
+    return std::max(1, n_full) * ((CH + threads - 1) / threads) * rpn.rp.VEC <= 32 ? threads : whole;
+}
+
 // `totals`: further requests whose destination holds one element and whose root is [scalar arithmetic over] one full
 // reduction of an expression with one value per row of `dom` (the mean of the row losses next to the gradient of a
 // cross-entropy). They ride along in the same launch: every workgroup publishes the combination of its rows' values,
@@ -760,7 +788,11 @@ bool try_row(const std::vector<DestSpec>& specs, const Domain& dom, const std::v
         // and it saves the shuffles: [1048576, 64] sum 41 us against 50 us)
         bool writes_rows = false;
         for (const Output& o : rpn.outputs) writes_rows = writes_rows || o.cls == Cls::FULL;
-        if (writes_rows) tpr = std::max(tpr, std::min(64, pow2ceil((int)std::max<int64_t>(1, CH))));
+        if (writes_rows) {
+            const int whole = std::min(64, pow2ceil((int)std::max<int64_t>(1, CH)));
+            tpr = std::max(tpr, whole);
+            if (nph >= 2 && CH <= 64 && dom.R * whole >= 65536) tpr = short_row_threads(rpn, CH, whole, n_full, big);
+        }
         if (rp.tail) tpr = std::max(tpr, rp.peel ? 8 : 4);  // one thread per element outside the whole vectors
         tpr = std::min(tpr, tpr_cap);
         int64_t ept = (CH + tpr - 1) / tpr;
