@@ -1238,6 +1238,18 @@ int dali_hip_sgemm_terms(int nterms, int transA, int transB, int M, int N, const
     return sgemm_rowmajor(nterms, transA != 0, transB != 0, M, N, K, A, ldas, B, ldbs, alpha, beta, C, ldc, true, row_map);
 }
 
+int dali_hip_conv2d_nhwc(int filters_gradient, int batch, int in_h, int in_w, int channels, int filters, int filter_h, int filter_w, int stride_h, int stride_w,
+                         const float* image, const float* other, float* result, int* taken) {
+    if (ensure_init()) return DALI_HIP_ERROR;
+    if (!image || !other || !result || !taken) return fail("dali_hip_conv2d_nhwc: NULL argument");
+    if (batch < 1 || in_h < 1 || in_w < 1 || channels < 1 || filters < 1 || filter_h < 1 || filter_w < 1 || stride_h < 1 || stride_w < 1)
+        return fail("dali_hip_conv2d_nhwc: extents and strides must be positive");
+    if (filter_h > in_h || filter_w > in_w) return fail("dali_hip_conv2d_nhwc: a %d x %d window does not fit a %d x %d image", filter_h, filter_w, in_h, in_w);
+    const int r = split_conv_nhwc(filters_gradient != 0, batch, in_h, in_w, channels, filters, filter_h, filter_w, stride_h, stride_w, image, other, result, device_cus());
+    *taken = r > 0;
+    return r < 0 ? DALI_HIP_ERROR : DALI_HIP_OK;
+}
+
 int dali_hip_lstm_step(int batch, int input, int hidden, const float* X, int ldx, const float* Hprev, int ldh,
                        const float* Cprev, const float* W, int ldw, const float* U, int ldu, const float* bias,
                        float* Cout, float* Hout) {

@@ -73,6 +73,50 @@ constexpr int kLowBytes = 4 * kPlaneBytes;         // m and l: two stages behind
 constexpr int kLow = 4 * kHighBytes, kLdsBytes = kLow + 2 * kLowBytes;
 constexpr int kMaxTerms = 8;
 
+// The convolutions of a channels-last image x [n, h, w, c] without padding, by their windows' positions (image, i, j) in order, position 0
+// at the image's first value: neighbours `step` values apart, rows of out_w of them `row` apart, images of out_h rows `image`.
+// A window's row kh is the run of `run` values from kh * line behind its position on.
+struct SplitConv {
+    int out_w, out_h, step, row, image, run, line;
+    unsigned hw, hw_m, w_m, run_m;  // exact divisions by out_h * out_w, out_w and run
+    int hw_s, w_s, run_s;
+    __device__ __forceinline__ int place(int k) const {
+        const int img = (int)sgemm_row_map_div((unsigned)k, hw_m, hw_s), rest = k - img * (int)hw, i = (int)sgemm_row_map_div((unsigned)rest, w_m, w_s);
+        return img * image + i * row + (rest - i * out_w) * step;
+    }
+    // value n of a window
+    __device__ __forceinline__ int within(int n) const {
+        const int kh = (int)sgemm_row_map_div((unsigned)n, run_m, run_s);
+        return kh * line + n - kh * run;
+    }
+};
+
+// consecutive positions
+struct Positions {
+    int i, j, at;
+    __device__ __forceinline__ void seek(const SplitConv& cv, int k) {
+        const int img = (int)sgemm_row_map_div((unsigned)k, cv.hw_m, cv.hw_s), rest = k - img * (int)cv.hw;
+        i = (int)sgemm_row_map_div((unsigned)rest, cv.w_m, cv.w_s);
+        j = rest - i * cv.out_w;
+        at = img * cv.image + i * cv.row + j * cv.step;
+    }
+    __device__ __forceinline__ void next(const SplitConv& cv) {
+        at += cv.step;
+        if (++j == cv.out_w) {
+            j = 0;
+            at += cv.row - cv.out_w * cv.step;
+            if (++i == cv.out_h) {
+                i = 0;
+                at += cv.image - cv.out_h * cv.row;
+            }
+        }
+    }
+};
+
+// What the operands are: matrices; for a convolution's result A is the image, row m the window at position m, a term per row of the
+// window; for the gradient of its filters B is the image, row k the window at position k
+enum Form { kPlain = 0, kWindows = 1, kFilters = 2 };
+
 struct SplitArgs {
     const float* A[kMaxTerms];
     const float* B[kMaxTerms];
@@ -86,6 +130,7 @@ struct SplitArgs {
     int slabs;        // of all terms together
     float* partials;  // shares > 1: [share][tile][16384], else unused
     SgemmRowMap map;
+    SplitConv cv;
 };
 
 __device__ __forceinline__ float lo_part(unsigned int pair) { return __uint_as_float(pair << 16); }
@@ -129,6 +174,27 @@ struct Loader {
     __device__ __forceinline__ void set_ld(int x0, int x_end, int ld) {
         const int x = min(x0 + row, x_end - 1);
         off = KROWS ? (unsigned)((x - x0) * ld + 8 * granule) : (unsigned)(8 * granule * ld + x);
+    }
+    // rows (columns) of windows: KROWS, from the window of the tile's first row; else from a window's first value
+    __device__ __forceinline__ void set_windows(const SplitConv& cv, int x0, int x_end) {
+        const int x = min(x0 + row, x_end - 1);
+        off = KROWS ? (unsigned)(cv.place(x) - cv.place(x0) + 8 * granule) : (unsigned)cv.within(x);
+    }
+    // eight windows' values (else)
+    __device__ __forceinline__ void fetch_windows(float* v, const float* p, const SplitConv& cv, Positions& at) const {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            v[j] = (p + at.at)[off];
+            at.next(cv);
+        }
+    }
+    __device__ __forceinline__ void fetch_windows_tail(float* v, const float* p, const SplitConv& cv, int k0, int left) const {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int k = 8 * __builtin_amdgcn_readfirstlane(granule) + j;
+            const float a = (p + cv.place(k0 + min(k, left - 1)))[off];
+            v[j] = k < left ? a : 0.0f;
+        }
     }
     // `p`: the tile's first row at the slab's first k (KROWS), the slab's first k (else)
     __device__ __forceinline__ void fetch(float* v, const float* p, int ld) const {
@@ -181,22 +247,24 @@ struct Loader {
 // Walks the slabs of the terms in order for the loads, which are the same instructions for every slab, so that the waits for one
 // slab leave the next ones' loads in flight: a partly filled last slab is fetched sixteen values of k ending at the last (what that
 // gets wrong is fetched again when it is cut), and behind the last slab of the share that one is fetched again.
-template <bool TA, bool TB>
+template <bool TA, bool TB, int F>
 struct Walk {
     Loader<!TA> a;
     Loader<TB> b;
+    Positions at;  // of the slab's windows (kFilters): of this wave's eight
     const float *pa, *pb;
     int term, left, lda, ldb, todo;  // left: values of k of the term from this slab on; todo: slabs to move on to
 
     __device__ __forceinline__ void enter(const SplitArgs& g, int k0, int m0, int n0) {
         lda = g.lda[term];
         ldb = g.ldb[term];
-        a.set_ld(m0, g.M, lda);
-        b.set_ld(n0, g.N, ldb);
+        if (F != kWindows) a.set_ld(m0, g.M, lda);
+        if (F != kFilters) b.set_ld(n0, g.N, ldb);
         left = g.K[term] - k0;
         k0 = min(k0, g.K[term] - kSlab);
-        pa = g.A[term] + (TA ? (size_t)k0 * lda : (size_t)m0 * lda + k0);
-        pb = g.B[term] + (TB ? (size_t)n0 * ldb + k0 : (size_t)k0 * ldb);
+        pa = g.A[term] + (F == kWindows ? (size_t)(g.cv.place(m0) + k0) : TA ? (size_t)k0 * lda : (size_t)m0 * lda + k0);
+        pb = g.B[term] + (F == kFilters ? (size_t)0 : TB ? (size_t)n0 * ldb + k0 : (size_t)k0 * ldb);
+        if (F == kFilters) at.seek(g.cv, k0 + 8 * __builtin_amdgcn_readfirstlane(b.granule));
     }
     __device__ __forceinline__ void start(const SplitArgs& g, int first_term, int k0, int count, int m0, int n0) {
         term = first_term;
@@ -206,14 +274,24 @@ struct Walk {
     // fetches the slab and moves on to the next
     __device__ __forceinline__ void fetch(const SplitArgs& g, float* va, float* vb, int m0, int n0) {
         a.fetch(va, pa, lda);
-        b.fetch(vb, pb, ldb);
+        Positions behind = at;
+        if (F == kFilters) b.fetch_windows(vb, pb, g.cv, behind);
+        else b.fetch(vb, pb, ldb);
         if (todo > 0) {
             --todo;
             left -= kSlab;
             if (left > 0) {
                 const int by = min(left, kSlab);
                 pa += TA ? (size_t)by * lda : (size_t)by;
-                pb += TB ? (size_t)by : (size_t)by * ldb;
+                if (F != kFilters) {
+                    pb += TB ? (size_t)by : (size_t)by * ldb;
+                } else if (by == kSlab) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) behind.next(g.cv);  // (the other half's windows)
+                    at = behind;
+                } else {
+                    at.seek(g.cv, g.K[term] - kSlab + 8 * __builtin_amdgcn_readfirstlane(b.granule));
+                }
             } else {
                 ++term;
                 enter(g, 0, m0, n0);
@@ -223,7 +301,7 @@ struct Walk {
 };
 
 // The same walk for the cutting, one to three slabs behind: tells the partly filled slabs.
-template <bool TA, bool TB>
+template <bool TA, bool TB, int F>
 struct Cutter {
     int term, left;
     __device__ __forceinline__ void start(const SplitArgs& g, int first_term, int k0) {
@@ -231,15 +309,16 @@ struct Cutter {
         left = g.K[term] - k0;
     }
     // the slab in `va`, `vb` with zeros behind the end of the term
-    __device__ __forceinline__ void settle(const SplitArgs& g, const Walk<TA, TB>& w, float* va, float* vb, int m0, int n0) {
+    __device__ __forceinline__ void settle(const SplitArgs& g, const Walk<TA, TB, F>& w, float* va, float* vb, int m0, int n0) {
         if (left > 0 && left < kSlab) {
             Loader<!TA> a = w.a;
             Loader<TB> b = w.b;
             const int lda = g.lda[term], ldb = g.ldb[term], k0 = g.K[term] - left;
-            a.set_ld(m0, g.M, lda);
-            b.set_ld(n0, g.N, ldb);
-            a.fetch_tail(va, g.A[term] + (TA ? (size_t)k0 * lda : (size_t)m0 * lda + k0), lda, left);
-            b.fetch_tail(vb, g.B[term] + (TB ? (size_t)n0 * ldb + k0 : (size_t)k0 * ldb), ldb, left);
+            if (F != kWindows) a.set_ld(m0, g.M, lda);
+            if (F != kFilters) b.set_ld(n0, g.N, ldb);
+            a.fetch_tail(va, g.A[term] + (F == kWindows ? (size_t)(g.cv.place(m0) + k0) : TA ? (size_t)k0 * lda : (size_t)m0 * lda + k0), lda, left);
+            if (F == kFilters) b.fetch_windows_tail(vb, g.B[term], g.cv, k0, left);
+            else b.fetch_tail(vb, g.B[term] + (TB ? (size_t)n0 * ldb + k0 : (size_t)k0 * ldb), ldb, left);
         }
         left -= kSlab;
         if (left <= 0 && term + 1 < g.nseg) left = g.K[++term];
@@ -270,7 +349,7 @@ __device__ __forceinline__ void store_result(const SplitArgs& g, int m, int n, f
     put(g, g.C + row * g.ldc + n, sum);
 }
 
-template <bool TA, bool TB>
+template <bool TA, bool TB, int F>
 __global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
     __shared__ __attribute__((aligned(16))) char lds[kLdsBytes];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -296,15 +375,17 @@ __global__ __launch_bounds__(256, 2) void sgemm_split_kernel(SplitArgs g) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = small[i][j] = floatx16{};
     const int wm = 64 * (wave >> 1), wn = 64 * (wave & 1);
-    Walk<TA, TB> w;
+    Walk<TA, TB, F> w;
     w.a.init(tid, m0, g.M, 0);
     w.b.init(tid, n0, g.N, 0);
+    if (F == kWindows) w.a.set_windows(g.cv, m0, g.M);
+    if (F == kFilters) w.b.set_windows(g.cv, n0, g.N);
     int first_term = 0, first_k = s_begin;
     while (first_term + 1 < g.nseg && first_k >= (g.K[first_term] + kSlab - 1) / kSlab) first_k -= (g.K[first_term++] + kSlab - 1) / kSlab;
     first_k *= kSlab;
     const int count = s_end - s_begin;
     w.start(g, first_term, first_k, count, m0, n0);
-    Cutter<TA, TB> c;
+    Cutter<TA, TB, F> c;
     c.start(g, first_term, first_k);
     float va[8], vb[8];
     const int ra = lds_offset(wm + (lane & 31), lane >> 5), rb = lds_offset(wn + (lane & 31), lane >> 5) + kPlaneBytes;
@@ -493,14 +574,65 @@ __global__ __launch_bounds__(256) void sgemm_split_fold(SplitArgs g) {
         if (m + v < g.M) store_result(g, m + v, n, sum[v]);
 }
 
+// The number of shares of the inner extent, 0 where the fp32 kernels at `fp32_rate` (TFLOP/s times 10^6; over whole 64x64 tiles) are estimated to be as fast
+// with what `g` describes, `beside`: and with what that form does besides, in microseconds.
+int choose_shares(const SplitArgs& g, int cus, double fp32_rate, bool long_rate, double beside = 0.0) {
+    const long tiles = (long)g.tiles_m * g.tiles_n;
+    // Whether and in how many shares, by estimated microseconds. Workgroups that share a compute unit pass a slab each in 0.8 us, one alone in
+    // 1.0; starting and ending a tile costs four slabs; adding shares up costs a launch and a read of them. The fp32 kernels by their
+    // rate over whole 64x64 tiles, in TFLOP/s: 76 where several terms or a row map leave them the register-staged kernel (measured 68 to 94); 135
+    // where their loads write LDS and up to four rounds of 64x64 tiles fill the chip (117 to 141); 115 over long inner extents, where they
+    // cut what does not fill a round into shares (117 to 136 at 1.4 to 2.4 tiles a compute unit); 112 else (45 to 145: operands off 16 bytes and rounds
+    // that are not full are the slow ones). Measured, us here / there, in the orders NN NT TN TT:
+    //   one 128x128 tile a compute unit, refused: 2048^2 over 512 39 38 40 38 / 37 36 35 36, over 1024 69 68 69 67 / 65 65 63 64; 1024^2 over 4096
+    //     63 62 63 63 / 64 61 63 61; [1883,10136] against [4486,10136] (NT) 1485 / 1411; [256,4096] over 512 24 24 24 24 / 11 11 11 11
+    //   two: [2048,4096] over 256 35 34 35 35 / 37 38 36 38, over 1024 107 105 106 106 / 124 126 122 125
+    //   three: [3072,4096] over 256 52 51 52 51 / 53 54 53 54, over 1024 161 160 163 160 / 185 185 180 185, over 4096 605 599 612 598 / 711 713 698 713
+    //   five: [4096,5120] over 256 79 78 80 79 / 87 88 85 87, over 1024 260 254 260 256 / 310 311 301 309
+    //   2.4 tiles, off 16 bytes: [573,15415] over 2683 395 397 400 396 / 581 589 910 900
+    //   shares: [256,1024] over 32000 110 108 110 110 / 131 129 132 129; [576,128] over 93312 116 114 108 110 / 118 116 119 116
+    //   rows of a convolution: [100352,128] over 3 x 192 122 / 166, [3136,256] over 3 x 384 30 / 27 (refused)
+    const int most = (int)(kWorkspacePartialBytes / (kTile * kTile * sizeof(float)) / tiles);
+    auto estimate = [&](int sh) {
+        const long per_cu = (tiles * sh + cus - 1) / cus;
+        const double slabs = (double)g.slabs / sh + 4.0;
+        return (per_cu < 2 ? slabs : 0.8 * (double)per_cu * slabs) + (sh > 1 ? 4.0 + 0.013 * (double)(tiles * sh) : 0.0);
+    };
+    int shares = 1;
+    for (int sh = 2; sh <= most && sh * 8 <= g.slabs; ++sh)
+        if (estimate(sh) < estimate(shares)) shares = sh;
+    if (long_rate && shares == 1 && g.K[0] >= 2048) fp32_rate = 115e6;
+    double flops = 0.0;
+    for (int s = 0; s < g.nseg; ++s) flops += 2.0 * ((g.M + 63) / 64 * 64) * ((g.N + 63) / 64 * 64) * (double)g.K[s];
+    if (estimate(shares) > 0.97 * (flops / fp32_rate + beside)) return 0;
+    return (long)g.slabs * (shares + 1) < (1L << 31) ? shares : 0;
+}
+
+int launch_split(SplitArgs& g, void (*kernel)(SplitArgs)) {
+    const long tiles = (long)g.tiles_m * g.tiles_n;
+    g.partials = (float*)(workspace() + kWorkspaceCounterBytes);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(tiles * g.shares)), dim3(256), 0, stream(), g);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && g.shares > 1) {
+        hipLaunchKernelGGL(sgemm_split_fold, dim3((unsigned)(tiles * 16)), dim3(256), 0, stream(), g);
+        e = hipGetLastError();
+    }
+    if (e != hipSuccess) return fail("sgemm launch failed: %s", hipGetErrorString(e));
+    return 1;
+}
+
+bool split_enabled(int cus) {
+    static const int enabled = getenv("DALI_HIP_GEMM_SPLIT") ? atoi(getenv("DALI_HIP_GEMM_SPLIT")) : 1;
+    return enabled && cus >= 8;
+}
+
 }  // namespace
 
 int sgemm_split(bool ta, bool tb, int M, int N, int nseg, const int* K, const float* const* A, const int* lda, const float* const* B, const int* ldb, float alpha,
                 float beta, float* C, int ldc, const SgemmRowMap& map, int cus) {
-    static const int enabled = getenv("DALI_HIP_GEMM_SPLIT") ? atoi(getenv("DALI_HIP_GEMM_SPLIT")) : 1;
     // (A sum of two products keeps the order of summation that the fused LSTM step has. What a pair stands for is not known here: two large
     // products that have nothing to do with a cell, or two filter rows of a convolution, stay on the fp32 kernels with it.)
-    if (!enabled || cus < 8 || nseg < 1 || nseg > kMaxTerms || nseg == 2 || M <= 64 || N <= 64 || K[0] <= 64) return 0;
+    if (!split_enabled(cus) || nseg < 1 || nseg > kMaxTerms || nseg == 2 || M <= 64 || N <= 64 || K[0] <= 64) return 0;
     SplitArgs g = {};
     for (int s = 0; s < nseg; ++s) {
         // offsets within a slab are 32-bit
@@ -525,51 +657,84 @@ int sgemm_split(bool ta, bool tb, int M, int N, int nseg, const int* K, const fl
     g.tiles_n = (N + kTile - 1) / kTile;
     const long tiles = (long)g.tiles_m * g.tiles_n;
     if (tiles > (1L << 24)) return 0;
-    // Whether and in how many shares, by estimated microseconds. Workgroups that share a compute unit pass a slab each in 0.8 us, one alone in
-    // 1.0; starting and ending a tile costs four slabs; adding shares up costs a launch and a read of them. The fp32 kernels by their
-    // rate over whole 64x64 tiles, in TFLOP/s: 76 where several terms or a row map leave them the register-staged kernel (measured 68 to 94); 135
-    // where their loads write LDS and up to four rounds of 64x64 tiles fill the chip (117 to 141); 115 over long inner extents, where they
-    // cut what does not fill a round into shares (117 to 136 at 1.4 to 2.4 tiles a compute unit); 112 else (45 to 145: operands off 16 bytes and rounds
-    // that are not full are the slow ones). Measured, us here / there, in the orders NN NT TN TT:
-    //   one 128x128 tile a compute unit, refused: 2048^2 over 512 39 38 40 38 / 37 36 35 36, over 1024 69 68 69 67 / 65 65 63 64; 1024^2 over 4096
-    //     63 62 63 63 / 64 61 63 61; [1883,10136] against [4486,10136] (NT) 1485 / 1411; [256,4096] over 512 24 24 24 24 / 11 11 11 11
-    //   two: [2048,4096] over 256 35 34 35 35 / 37 38 36 38, over 1024 107 105 106 106 / 124 126 122 125
-    //   three: [3072,4096] over 256 52 51 52 51 / 53 54 53 54, over 1024 161 160 163 160 / 185 185 180 185, over 4096 605 599 612 598 / 711 713 698 713
-    //   five: [4096,5120] over 256 79 78 80 79 / 87 88 85 87, over 1024 260 254 260 256 / 310 311 301 309
-    //   2.4 tiles, off 16 bytes: [573,15415] over 2683 395 397 400 396 / 581 589 910 900
-    //   shares: [256,1024] over 32000 110 108 110 110 / 131 129 132 129; [576,128] over 93312 116 114 108 110 / 118 116 119 116
-    //   rows of a convolution: [100352,128] over 3 x 192 122 / 166, [3136,256] over 3 x 384 30 / 27 (refused)
-    const int most = (int)(kWorkspacePartialBytes / (kTile * kTile * sizeof(float)) / tiles);
-    auto estimate = [&](int sh) {
-        const long per_cu = (tiles * sh + cus - 1) / cus;
-        const double slabs = (double)g.slabs / sh + 4.0;
-        return (per_cu < 2 ? slabs : 0.8 * (double)per_cu * slabs) + (sh > 1 ? 4.0 + 0.013 * (double)(tiles * sh) : 0.0);
-    };
-    g.shares = 1;
-    for (int sh = 2; sh <= most && sh * 8 <= g.slabs; ++sh)
-        if (estimate(sh) < estimate(g.shares)) g.shares = sh;
     bool direct = true;  // the loads of the fp32 kernels can write LDS
     for (int s = 0; s < nseg; ++s) direct = direct && lda[s] % 4 == 0 && ldb[s] % 4 == 0 && (((uintptr_t)A[s] | (uintptr_t)B[s]) & 15) == 0;
     const long tiles64 = (long)((M + 63) / 64) * ((N + 63) / 64), rounds64 = (tiles64 + cus - 1) / cus;
     const bool fills = tiles <= cus && (double)tiles64 >= 0.95 * (double)(rounds64 * cus);
-    const double fp32_rate = nseg > 2 || map.on ? 76e6 : !direct ? 112e6 : fills ? 135e6 : g.shares == 1 && K[0] >= 2048 ? 115e6 : 112e6;
-    double flops = 0.0;
-    for (int s = 0; s < nseg; ++s) flops += 2.0 * ((M + 63) / 64 * 64) * ((N + 63) / 64 * 64) * (double)K[s];
-    if (estimate(g.shares) > 0.97 * flops / fp32_rate) return 0;
-    if ((long)g.slabs * (g.shares + 1) >= (1L << 31)) return 0;
-    g.partials = (float*)(workspace() + kWorkspaceCounterBytes);
-    const dim3 grid((unsigned)(tiles * g.shares));
-    if (!ta && !tb) hipLaunchKernelGGL((sgemm_split_kernel<false, false>), grid, dim3(256), 0, stream(), g);
-    else if (ta && !tb) hipLaunchKernelGGL((sgemm_split_kernel<true, false>), grid, dim3(256), 0, stream(), g);
-    else if (!ta && tb) hipLaunchKernelGGL((sgemm_split_kernel<false, true>), grid, dim3(256), 0, stream(), g);
-    else hipLaunchKernelGGL((sgemm_split_kernel<true, true>), grid, dim3(256), 0, stream(), g);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && g.shares > 1) {
-        hipLaunchKernelGGL(sgemm_split_fold, dim3((unsigned)(tiles * 16)), dim3(256), 0, stream(), g);
-        e = hipGetLastError();
+    const bool staged = nseg > 2 || map.on;
+    g.shares = choose_shares(g, cus, staged ? 76e6 : !direct ? 112e6 : fills ? 135e6 : 112e6, !staged && direct && !fills);
+    if (g.shares == 0) return 0;
+    if (!ta && !tb) return launch_split(g, sgemm_split_kernel<false, false, kPlain>);
+    if (ta && !tb) return launch_split(g, sgemm_split_kernel<true, false, kPlain>);
+    if (!ta && tb) return launch_split(g, sgemm_split_kernel<false, true, kPlain>);
+    return launch_split(g, sgemm_split_kernel<true, true, kPlain>);
+}
+
+// The convolution of a channels-last image [n, h, w, c] with filters [f, fh, fw, c], without padding, and the gradient of its filters, as products whose
+// one operand is the image itself, read window by window: no patch matrix is written or read, and no padded copy of the image. `result`
+// as the matrix product lays it out: [n, out_h, out_w, f] (filters_gradient: [f, fh, fw, c], from `out` [n, out_h, out_w, f]). Taken where the rule above takes
+// the product of that size. 1: launched; 0: not a case for it (form the patch matrix); -1: failure (message set).
+// What the product alone takes is left: us, image padded or patch matrix formed first / here, [32,56,56,64] with 128 filters of 3x3 147 / 107 and gradient 169 / 112, at stride
+// 2 58 / 45 and 67 / 45; [8,64,64,33], 100 of 5x5 120 / 65 and 216 / 59; [32,56,56,128], 128 of 3x3 248 / 190 and 280 / 180; [64,28,28,256], 256 of 1x1 95 / 65 and 75 / 64.
+int split_conv_nhwc(bool filters_gradient, int n, int h, int w, int c, int f, int fh, int fw, int stride_h, int stride_w, const float* image, const float* other,
+                    float* result, int cus) {
+    const int oh = (h - fh) / stride_h + 1, ow = (w - fw) / stride_w + 1;
+    const long positions = (long)n * oh * ow, run = (long)fw * c;
+    if (!split_enabled(cus) || h < fh || w < fw || (long)n * h * w * c >= (1L << 30) || positions * f >= (1L << 30) || (long)f * fh * run >= (1L << 30)) return 0;
+    SplitArgs g = {};
+    SplitConv& cv = g.cv;
+    cv.out_w = ow;
+    cv.out_h = oh;
+    cv.step = stride_w * c;
+    cv.row = stride_h * w * c;
+    cv.image = h * w * c;
+    cv.run = (int)run;
+    cv.line = w * c;
+    auto divide_by = [](unsigned d, unsigned* m, int* shift) {
+        int s = 0;
+        while ((1ull << s) < d) ++s;
+        *m = (unsigned)(((1ull << (31 + s)) + d - 1) / d);
+        *shift = s;
+    };
+    cv.hw = (unsigned)(oh * ow);
+    divide_by(cv.hw, &cv.hw_m, &cv.hw_s);
+    divide_by((unsigned)ow, &cv.w_m, &cv.w_s);
+    divide_by((unsigned)run, &cv.run_m, &cv.run_s);
+    if (filters_gradient) {
+        g.nseg = 1;
+        g.A[0] = other;
+        g.lda[0] = f;
+        g.B[0] = image;
+        g.K[0] = (int)positions;
+        g.M = f;
+        g.N = fh * (int)run;
+    } else {
+        if (fh > kMaxTerms) return 0;
+        g.nseg = fh;
+        for (int s = 0; s < fh; ++s) {
+            g.A[s] = image + (size_t)s * cv.line;
+            g.B[s] = other + (size_t)s * run;
+            g.ldb[s] = fh * (int)run;
+            g.K[s] = (int)run;
+        }
+        g.M = (int)positions;
+        g.N = f;
     }
-    if (e != hipSuccess) return fail("sgemm launch failed: %s", hipGetErrorString(e));
-    return 1;
+    if (g.M <= 64 || g.N <= 64 || g.K[0] <= 64) return 0;
+    for (int s = 0; s < g.nseg; ++s) g.slabs += (g.K[s] + kSlab - 1) / kSlab;
+    g.C = result;
+    g.ldc = g.N;
+    g.alpha = 1.0f;
+    g.tiles_m = (g.M + kTile - 1) / kTile;
+    g.tiles_n = (g.N + kTile - 1) / kTile;
+    if ((long)g.tiles_m * g.tiles_n > (1L << 24)) return 0;
+    // what it stands in for: a launch that forms a patch matrix, written and read at about 4.5 TB/s, and a product (off 16 bytes at 40 to 60 TFLOP/s); at stride 1 and
+    // whole vectors of channels a padded copy of the image and a sum of products
+    const double product = c % 4 == 0 && f % 4 == 0 ? 112e6 : 60e6, patches = 5.0 + 8.0 * (double)positions * (fh * run) / 4.5e6;
+    const bool summed = !filters_gradient && stride_h == 1 && stride_w == 1 && c % 4 == 0;
+    g.shares = choose_shares(g, cus, summed ? 76e6 : product, false, summed ? 5.0 + 8.0 * n * h * w * c / 4.5e6 : patches);
+    if (g.shares == 0) return 0;
+    return launch_split(g, filters_gradient ? sgemm_split_kernel<true, false, kFilters> : sgemm_split_kernel<false, true, kWindows>);
 }
 
 }  // namespace dali_hip

@@ -1278,6 +1278,15 @@ static void check_ndim4(const char* name, const char* array_name, const Array& a
     DALI_ASSERT(a.ndim() == 4, make_message(name, "'s ", array_name, " must be 4 dimensional but got ", array_name, " with ndim = ", a.ndim(), "."));
 }
 
+// Whether a convolution of these sizes may be read from the image window by window (dali_hip_conv2d_nhwc, which judges what is left): channels-last, no
+// padding, and as many operations as a large product has. DALI_HIP_CONV_IM2COL=1 keeps the two-step form.
+static bool convolves_by_windows(const ConvFunctionInfo& info, const std::string& data_format, const Array& a, const Array& b) {
+    static const bool two_step = getenv("DALI_HIP_CONV_IM2COL") != nullptr;
+    return !two_step && !dry_run() && data_format == "NHWC" && a.ndim() == 4 && b.ndim() == 4 && a.dtype() == DTYPE_FLOAT && b.dtype() == DTYPE_FLOAT && info.padding_h == 0 &&
+           info.padding_w == 0 && info.odd_padding_h == 0 && info.odd_padding_w == 0 && info.out_h >= 1 && info.out_w >= 1 &&
+           2.0 * info.batch_size * info.out_h * info.out_w * info.out_channels * info.filter_h * info.filter_w * info.in_channels >= 1e9;
+}
+
 // dali/array/op/conv.cpp:223-276: filters [out, ...] flattened to a matrix times the patch matrix
 Array conv2d(const Array& input, const Array& filters, int stride_h, int stride_w, PADDING_T padding, const std::string& data_format) {
     DALI_ASSERT(input.ndim() == 3 || input.ndim() == 4, make_message("Input argument to conv2d must be 3D or 4D (got input.ndim=", input.ndim(), ")."));
@@ -1286,6 +1295,11 @@ Array conv2d(const Array& input, const Array& filters, int stride_h, int stride_
     check_data_format(data_format, &n_dim, &c_dim, &h_dim, &w_dim);
     check_nchw_or_nhwc("conv2d", data_format);
     ConvFunctionInfo info = compute_conv2d_info(with_batch_axis(input.shape(), n_dim), filters.shape(), stride_h, stride_w, padding, data_format);
+    Array by_windows;
+    if (convolves_by_windows(info, data_format, input, filters) &&
+        conv2d_windows_nhwc(false, input, filters, {info.batch_size, info.out_h, info.out_w, info.out_channels}, info.out_channels, info.filter_h, info.filter_w, stride_h, stride_w,
+                            &by_windows))
+        return by_windows;
     // channels-last, stride 1: no patch matrix (see conv2d_direct_nhwc); DALI_HIP_CONV_IM2COL=1 keeps the two-step form
     static const bool two_step = getenv("DALI_HIP_CONV_IM2COL") != nullptr;
     if (!two_step && !dry_run() && data_format == "NHWC" && stride_h == 1 && stride_w == 1 && input.ndim() == 4 && input.dtype() == DTYPE_FLOAT &&
@@ -1336,6 +1350,10 @@ Array conv2d_backward_filters(Array input, Array out_dw, int stride_h, int strid
     check_nchw_or_nhwc("conv2d_backward_filters", data_format);
     DALI_ASSERT(filters_shape.size() == 4, make_message("conv2d_backward_filters's filters_shape must be of size 4, but got ", shape_str(filters_shape), "."));
     ConvFunctionInfo info = compute_conv2d_info(input.shape(), filters_shape, stride_h, stride_w, padding, data_format);
+    Array by_windows;
+    if (convolves_by_windows(info, data_format, input, out_dw) && out_dw.shape() == std::vector<int>{info.batch_size, info.out_h, info.out_w, info.out_channels} &&
+        conv2d_windows_nhwc(true, input, out_dw, filters_shape, info.out_channels, info.filter_h, info.filter_w, stride_h, stride_w, &by_windows))
+        return by_windows;
     Array patches_t = im2col(input, info.filter_h, info.filter_w, stride_h, stride_w, info.padding_h, info.padding_w,
                              info.padding_h + info.odd_padding_h, info.padding_w + info.odd_padding_w, data_format).transpose();
     if (data_format == "NCHW") {

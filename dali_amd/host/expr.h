@@ -112,6 +112,8 @@ void gru_recurrent_persistent(const Array& pre, const Array& U, const Array& h0,
 void softmax_axis_launch(const Array& x, const Array& out, long long outer, int extent, long long inner);
 // stride-1 convolution of a dense float NHWC image [N,H,W,C] (C a multiple of 4) with filters [O,fh,fw,C], fh <= 8:
 // one padding copy and one multi-term product, no patch matrix; returns [N, out_h, out_w, O]
+bool conv2d_windows_nhwc(bool filters_gradient, const Array& image, const Array& other, const std::vector<int>& result_shape, int f, int fh, int fw, int stride_h, int stride_w,
+                         Array* result);
 Array conv2d_direct_nhwc(const Array& x, const Array& filters, int pad_top, int pad_left, int pad_bottom, int pad_right);
 // column numbers of the k best entries of every row of a [rows, cols] matrix, best first (evaluates its argument)
 Array topk_rows(const Array& x2d, int k, bool largest, bool ties_by_descending_column);

@@ -487,9 +487,43 @@ static Array conv2d_nhwc_direct(const Array& x_in, const Array& filters_in, int 
     return out;
 }
 
+// The convolution of a channels-last image without padding, or the gradient of its filters, read from the image window by window
+// (dali_hip_conv2d_nhwc). False where the library does not take the size.
+static bool conv2d_nhwc_by_windows(bool filters_gradient, const Array& image_in, const Array& other_in, const std::vector<int>& result_shape, int f, int fh, int fw, int stride_h,
+                                   int stride_w, Array* result) {
+    Array image = dense_buffer(image_in), other = dense_buffer(other_in);
+    const std::vector<int> s = image.shape();
+    Array out(result_shape, DTYPE_FLOAT);
+    const float* ip = (const float*)image.device_ptr();
+    const float* op_ = (const float*)other.device_ptr();
+    float* rp = (float*)out.device_ptr(memory::AM_OVERWRITE);
+    auto issue = [=]() {
+        int taken = 0;
+        check_hip(dali_hip_conv2d_nhwc(filters_gradient, s[0], s[1], s[2], s[3], f, fh, fw, stride_h, stride_w, ip, op_, rp, &taken), "convolution product");
+        return taken != 0;
+    };
+    if (!issue()) return false;
+    jit_stats().gemms_launched++;
+    if (g_recording) {
+        note_recorded_write(out.expression()->memory);
+        std::vector<Array> keep = {image, other, out};
+        g_recording->push_back([=]() {
+            (void)keep;
+            issue();
+        });
+    }
+    *result = out;
+    return true;
+}
+
 }  // namespace jit
 
 using namespace jit;
+
+bool conv2d_windows_nhwc(bool filters_gradient, const Array& image, const Array& other, const std::vector<int>& result_shape, int f, int fh, int fw, int stride_h, int stride_w,
+                         Array* result) {
+    return conv2d_nhwc_by_windows(filters_gradient, image, other, result_shape, f, fh, fw, stride_h, stride_w, result);
+}
 
 Array conv2d_direct_nhwc(const Array& x, const Array& filters, int pad_top, int pad_left, int pad_bottom, int pad_right) {
     return conv2d_nhwc_direct(x, filters, pad_top, pad_left, pad_bottom, pad_right);

@@ -249,6 +249,14 @@ int dali_hip_sgemm_pair(int transB1, int transA1, int transB2, int transA2, int 
 int dali_hip_sgemm_terms(int nterms, int transA, int transB, int M, int N, const int* K, const float* const* A, int lda,
                          const float* const* B, int ldb, float alpha, float beta, float* C, int ldc, const int* row_map);
 
+/* Convolution of a channels-last image [batch, in_h, in_w, channels] without padding, or the gradient of its filters, as one product that reads the
+ * image window by window (no patch matrix, no padded copy). filters_gradient 0: other = filters [filters, filter_h, filter_w, channels], result
+ * [batch, out_h, out_w, filters]; 1: other = the gradient of that result, result = that of the filters. out = (in - filter) / stride + 1.
+ * *taken = 0: nothing was launched, the size is not one for this form (small products, more than 8 filter rows): use im2col and a product.
+ * Replaces im2col + op::dot (dali/array/op/conv.cpp:253-272, 369-392) for NHWC. */
+int dali_hip_conv2d_nhwc(int filters_gradient, int batch, int in_h, int in_w, int channels, int filters, int filter_h, int filter_w, int stride_h, int stride_w,
+                         const float* image, const float* other, float* result, int* taken);
+
 /*
  * One LSTM cell step in a single launch: pre = X[batch, input] . W[input, 4 hidden] + Hprev[batch, hidden] .
  * U[hidden, 4 hidden] (row-major, gates packed i, f, o, g along the columns), then per element
