@@ -27,6 +27,11 @@ def _load():
 
 
 hip, front = _load()
+try:
+    from . import _bind  # noqa: F401  (built on libdali_front)
+except ImportError as e:
+    raise ImportError("native library dali_amd/_bind.so is missing or does not load (%s): build it with `python -c 'import __graft_entry__ as g; g.build()'` "
+                      "from the repository root (there is no fallback path)" % e)
 
 H = C.c_void_p
 _i = C.c_int

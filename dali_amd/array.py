@@ -3,7 +3,7 @@ import ctypes as C
 
 import numpy as np
 
-from ._native import front, fe_error
+from ._native import _bind, front, fe_error, DaliError
 
 DTYPE_FLOAT, DTYPE_DOUBLE, DTYPE_INT32 = 0, 1, 2
 _NP = {DTYPE_FLOAT: np.float32, DTYPE_DOUBLE: np.float64, DTYPE_INT32: np.int32}
@@ -34,16 +34,10 @@ def as_array(x):
     return Array.from_numpy(np.asarray(x))
 
 
-class Array(object):
+class Array(_bind.Handle):
+    """Shape, strides, dtype, evaluation and the arithmetic operators are native (dali_amd/host/python_bind.cpp)."""
+
     __array_priority__ = 100
-
-    def __init__(self, handle):
-        self._h = handle
-
-    def __del__(self):
-        h, self._h = getattr(self, "_h", None), None
-        if h and front is not None:
-            front.dali_fe_release(h)
 
     # ---- construction
     @staticmethod
@@ -74,32 +68,6 @@ class Array(object):
         return _wrap(front.dali_fe_zeros(s, nd, dtype), "zeros")
 
     # ---- inspection
-    @property
-    def ndim(self):
-        return front.dali_fe_ndim(self._h)
-
-    @property
-    def shape(self):
-        nd = self.ndim
-        out = (C.c_int * max(1, nd))()
-        front.dali_fe_shape(self._h, out)
-        return tuple(out[i] for i in range(nd))
-
-    @property
-    def dtype(self):
-        return front.dali_fe_dtype(self._h)
-
-    @property
-    def strides(self):
-        nd = self.ndim
-        out = (C.c_int * max(1, nd))()
-        front.dali_fe_strides(self._h, out)
-        return tuple(out[i] for i in range(nd))
-
-    @property
-    def offset(self):
-        return front.dali_fe_offset(self._h)
-
     def is_buffer(self):
         return bool(front.dali_fe_is_buffer(self._h))
 
@@ -110,8 +78,7 @@ class Array(object):
     def transpose(self, *axes):
         if len(axes) == 1 and isinstance(axes[0], (tuple, list)):
             axes = axes[0]
-        a, n = _ints(axes)
-        return _wrap(front.dali_fe_transpose(self._h, a, n), "transpose")
+        return _bind.transpose(self, axes)
 
     @property
     def T(self):
@@ -169,24 +136,16 @@ class Array(object):
         return out
 
     # ---- evaluation
-    def eval(self):
-        if front.dali_fe_eval(self._h) != 0:
-            raise fe_error("eval")
-        return self
-
     def numpy(self):
         out = np.empty(self.shape, dtype=_NP[self.dtype])
         if front.dali_fe_to_host(self._h, out.ctypes.data_as(C.c_void_p)) != 0:
             raise fe_error("to_host")
         return out
 
-    def device_ptr(self):
-        p = front.dali_fe_device_ptr(self._h)
-        if not p:
-            raise fe_error("device_ptr")
-        return p
-
     def assign(self, other, operator_t=0):
+        if type(operator_t) is int:
+            _bind.assign(self, operator_t, other)
+            return self
         other = as_array(other)
         if front.dali_fe_assign(self._h, operator_t, other._h) != 0:
             raise fe_error("assign")
@@ -215,43 +174,7 @@ class Array(object):
         from . import op
         return op.gather_from_rows(self, indices)
 
-    # ---- arithmetic sugar
-    def __add__(self, o):
-        from . import op
-        return op.add(self, o)
-
-    def __radd__(self, o):
-        from . import op
-        return op.add(o, self)
-
-    def __sub__(self, o):
-        from . import op
-        return op.subtract(self, o)
-
-    def __rsub__(self, o):
-        from . import op
-        return op.subtract(o, self)
-
-    def __mul__(self, o):
-        from . import op
-        return op.eltmul(self, o)
-
-    def __rmul__(self, o):
-        from . import op
-        return op.eltmul(o, self)
-
-    def __truediv__(self, o):
-        from . import op
-        return op.eltdiv(self, o)
-
-    def __rtruediv__(self, o):
-        from . import op
-        return op.eltdiv(o, self)
-
-    def __neg__(self):
-        from . import op
-        return op.eltmul(-1, self)
-
+    # ---- reductions and products
     def sum(self, axes=None, keepdims=False):
         from . import op
         return op.sum(self, axes, keepdims)
@@ -279,6 +202,9 @@ class Array(object):
     def dot(self, other):
         from . import op
         return op.dot(self, other)
+
+
+_bind.register(Array, DaliError, as_array)
 
 
 def eval_together(arrays):

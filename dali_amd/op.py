@@ -1,28 +1,24 @@
 """``op``: the lazy operator factories (``dali/array/op.h`` of the reference)."""
 import ctypes as C
 
-from ._native import front, fe_error, DaliError
+from ._native import _bind, front, fe_error, DaliError
 from .array import Array, as_array, _ints, _wrap, DTYPE_FLOAT, DTYPE_DOUBLE, DTYPE_INT32  # noqa: F401
 
 
 def elementwise(functor_name, a, b=None):
-    a = as_array(a)
-    if b is None:
-        return _wrap(front.dali_fe_unary(functor_name.encode(), a._h), functor_name)
-    b = as_array(b)
-    return _wrap(front.dali_fe_binary(functor_name.encode(), a._h, b._h), functor_name)
+    return _bind.unary(functor_name, a) if b is None else _bind.binary(functor_name, a, b)
 
 
 def _unary(name):
     def f(x):
-        return elementwise(name, x)
+        return _bind.unary(name, x)
     f.__name__ = name
     return f
 
 
 def _binary(name):
     def f(a, b):
-        return elementwise(name, a, b)
+        return _bind.unary(name, a) if b is None else _bind.binary(name, a, b)
     f.__name__ = name
     return f
 
@@ -84,13 +80,7 @@ def astype(a, dtype):
 
 
 def _reduce(reducer, x, axes, keepdims):
-    x = as_array(x)
-    if axes is None:
-        return _wrap(front.dali_fe_all_reduce(reducer.encode(), x._h), reducer)
-    if isinstance(axes, int):
-        axes = [axes]
-    a, n = _ints(axes)
-    return _wrap(front.dali_fe_axis_reduce(reducer.encode(), x._h, a, n, 1 if keepdims else 0), reducer)
+    return _bind.all_reduce(reducer, x) if axes is None else _bind.axis_reduce(reducer, x, axes, keepdims)
 
 
 def sum(x, axes=None, keepdims=False):
@@ -120,6 +110,8 @@ def mean(x, axes=None, keepdims=False):
 
 
 def _arg(reducer, x, axis):
+    if type(axis) is int:
+        return _bind.arg_axis_reduce(reducer, x, axis, "arg " + reducer)
     x = as_array(x)
     if axis is None:
         return _wrap(front.dali_fe_arg_all_reduce(reducer.encode(), x._h), "arg " + reducer)
@@ -137,6 +129,8 @@ def argmin(x, axis=None):
 # Converted operands are bound to local names for the duration of each native
 # call: a temporary Array would release its handle before the call reads it.
 def softmax(x, axis=-1):
+    if type(axis) is int:
+        return _bind.softmax(x, axis)
     x = as_array(x)
     return _wrap(front.dali_fe_softmax(x._h, axis), "softmax")
 
@@ -150,13 +144,11 @@ def softmax_naive(x, axis=-1):
 
 def gather(source, indices):
     """source[indices[...], ...]; assigning to the lazy result scatters into ``source``."""
-    source, indices = as_array(source), as_array(indices)
-    return _wrap(front.dali_fe_gather(source._h, indices._h), "gather")
+    return _bind.gather(source, indices)
 
 
 def gather_from_rows(source, indices):
-    source, indices = as_array(source), as_array(indices)
-    return _wrap(front.dali_fe_gather_from_rows(source._h, indices._h), "gather_from_rows")
+    return _bind.gather_from_rows(source, indices)
 
 
 def one_hot(indices, depth, on_value, off_value):
@@ -165,8 +157,7 @@ def one_hot(indices, depth, on_value, off_value):
 
 
 def dot(a, b):
-    a, b = as_array(a), as_array(b)
-    return _wrap(front.dali_fe_dot(a._h, b._h), "dot")
+    return _bind.dot(a, b)
 
 
 def inner(a, b):
@@ -222,20 +213,12 @@ def tensordot(a, b, axes):
 
 def softmax_cross_entropy(logits, targets):
     """(mean loss, per-row loss, gradient) of the LSE-form softmax cross-entropy, evaluated together."""
-    outs = [C.c_void_p() for _ in range(3)]
-    logits, targets = as_array(logits), as_array(targets)
-    if front.dali_fe_softmax_cross_entropy(logits._h, targets._h, *[C.byref(o) for o in outs]) != 0:
-        raise fe_error("softmax_cross_entropy")
-    return tuple(Array(o.value) for o in outs)
+    return _bind.softmax_cross_entropy(logits, targets)
 
 
 def lstm_step(x, h, c, W, U, b):
     """One LSTM cell step; returns (c', h') already evaluated."""
-    outs = [C.c_void_p() for _ in range(2)]
-    keep = [as_array(v) for v in (x, h, c, W, U, b)]
-    if front.dali_fe_lstm_step(*[k._h for k in keep], *[C.byref(o) for o in outs]) != 0:
-        raise fe_error("lstm_step")
-    return tuple(Array(o.value) for o in outs)
+    return _bind.lstm_step(x, h, c, W, U, b)
 
 
 def lstm_sequence(xs, h0, c0, W, U, b):
