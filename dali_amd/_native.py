@@ -99,6 +99,7 @@ HIP_SYMBOLS = {
     "dali_hip_lstm_step": (_i, [_i, _i, _i, H, _i, H, _i, H, H, _i, H, _i, H, H, H]),
     "dali_hip_lstm_step_small": (_i, [_i, _i, _i, H, _i, H, _i, H, H, _i, H, _i, H, H, H]),
     "dali_hip_lstm_recurrent_persistent": (_i, [_i, _i, _i, H, H, _i, H, H, H, H]),
+    "dali_hip_lstm_recurrent_persistent_bias": (_i, [_i, _i, _i, H, H, H, _i, H, H, H, H]),
     "dali_hip_lstm_recurrent_persistent_supported": (_i, [_i, _i]),
     "dali_hip_gru_recurrent_persistent": (_i, [_i, _i, _i, H, H, _i, H, H, H]),
     "dali_hip_gru_recurrent_persistent_supported": (_i, [_i, _i]),

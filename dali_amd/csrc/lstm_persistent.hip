@@ -46,6 +46,7 @@ __device__ __forceinline__ float seq_expf(float x) {
 struct PersistentArgs {
     int T, B, H, HU, ldu;
     const float* pre;   // [T, B, 4H]
+    const float* bias;  // [4H], added to pre; may be null
     const float* U;     // [H, 4H], row stride ldu
     const float* h0;    // [B, H]
     const float* c0;    // [B, H]
@@ -154,6 +155,10 @@ __global__ __launch_bounds__(256) void lstm_persistent_kernel(PersistentArgs a) 
         if (owner) {
 #pragma unroll
             for (int gate = 0; gate < 4; ++gate) pre4[gate] = a.pre[((size_t)t * B + pb) * 4 * H + (size_t)gate * H + u0 + puu];
+            if (a.bias) {
+#pragma unroll
+                for (int gate = 0; gate < 4; ++gate) pre4[gate] += a.bias[(size_t)gate * H + u0 + puu];
+            }
         }
     };
     fetch_pre(0);
@@ -174,6 +179,15 @@ __global__ __launch_bounds__(256) void lstm_persistent_kernel(PersistentArgs a) 
         // every workgroup's pattern has reached memory before anybody's first h does
         if (tid == 0 && !wait_for(gridDim.x)) give_up = 1;
         __syncthreads();
+    }
+    // Up to 32 rows the values of the slice that this lane feeds to the products of every step stay in registers (more tiles of h leave no room for
+    // them: 48 rows 14.7 us a step, with them 16.1).
+    float ub[DATA_FLAGS ? KQ : 1][4];
+    if (DATA_FLAGS) {
+#pragma unroll
+        for (int q = 0; q < KQ; ++q)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) ub[q][c] = Us[(size_t)(wave * KW + 16 * q + 4 * kgrp + c) * P + arow];
     }
     for (int t = 0; t < a.T && !give_up; ++t) {
         const float* hp = t == 0 ? a.h0 : a.hs + (size_t)(t - 1) * B * H;
@@ -205,10 +219,12 @@ __global__ __launch_bounds__(256) void lstm_persistent_kernel(PersistentArgs a) 
 #pragma unroll
             for (int m = 0; m < MT; ++m) need[m] = true;
             // The waiting is done on one load per lane: a wave that fetched all its tiles again and again would multiply the
-            // traffic of the step (at 64 rows every workgroup reads 256 KiB of h) and slow the producers it waits for.
+            // traffic of the step (at 64 rows every workgroup reads 256 KiB of h) and slow the producers it waits for. It covers the first
+            // row over the wave's whole K range, so that it shows a value of every workgroup the wave depends on (sixteen rows over sixteen values
+            // of k, of four workgroups only, had the tiles fetched again and again: 32 steps of 16 rows of 1024 230 us, now 194, 8 rows of 512 159, now 118;
+            // fetching through the L2 after the wait was no faster, and a line that it takes too early stays old in it).
             while (polls < a.spin_limit) {
-                const int kb = wave * KW + 4 * kgrp;
-                const f4 probe = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(hrow, (arow * H + kb) * 4, 0, kPollLoad));
+                const f4 probe = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(hrow, 4 * lane < KW ? (wave * KW + 4 * lane) * 4 : 0x7ffffff0, 0, kPollLoad));
                 if (!__any(any_not_yet(probe))) break;
                 asm volatile("" ::: "memory");
                 __builtin_amdgcn_s_sleep(1);
@@ -246,7 +262,7 @@ __global__ __launch_bounds__(256) void lstm_persistent_kernel(PersistentArgs a) 
             const int kb = wave * KW + 16 * q + 4 * kgrp;
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                const float bv = Us[(size_t)(kb + c) * P + arow];  // B operand: row k of the slice, column lane % 16
+                const float bv = DATA_FLAGS ? ub[DATA_FLAGS ? q : 0][c] : Us[(size_t)(kb + c) * P + arow];  // B operand: row k of the slice, column lane % 16
 #pragma unroll
                 for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[q][m][c], bv, acc[m], 0, 0, 0);
             }
@@ -532,6 +548,11 @@ extern "C" int dali_hip_lstm_recurrent_persistent_supported(int batch, int hidde
 
 extern "C" int dali_hip_lstm_recurrent_persistent(int steps, int batch, int hidden, const float* pre, const float* U, int ldu, const float* h0,
                                                   const float* c0, float* hs, float* c_out) {
+    return dali_hip_lstm_recurrent_persistent_bias(steps, batch, hidden, pre, nullptr, U, ldu, h0, c0, hs, c_out);
+}
+
+extern "C" int dali_hip_lstm_recurrent_persistent_bias(int steps, int batch, int hidden, const float* pre, const float* bias, const float* U, int ldu, const float* h0,
+                                                       const float* c0, float* hs, float* c_out) {
     if (ensure_init()) return DALI_HIP_ERROR;
     if (steps < 1 || batch < 1 || hidden < 1) return fail("dali_hip_lstm_recurrent_persistent: steps, batch and hidden must be positive");
     if (!pre || !U || !h0 || !c0 || !hs || !c_out) return fail("dali_hip_lstm_recurrent_persistent: NULL argument");
@@ -541,7 +562,7 @@ extern "C" int dali_hip_lstm_recurrent_persistent(int steps, int batch, int hidd
         // rows 0 .. steps-2 of hs are overwritten while h0, c0 and pre are still being read
         const char *lo = (const char*)hs, *hi = lo + (size_t)steps * batch * hidden * sizeof(float);
         auto inside = [&](const void* p, size_t bytes) { return (const char*)p < hi && (const char*)p + bytes > lo; };
-        if (inside(h0, (size_t)batch * hidden * 4) || inside(c0, (size_t)batch * hidden * 4) || inside(pre, (size_t)steps * batch * hidden * 16))
+        if ((bias && inside(bias, (size_t)hidden * 16)) || inside(h0, (size_t)batch * hidden * 4) || inside(c0, (size_t)batch * hidden * 4) || inside(pre, (size_t)steps * batch * hidden * 16))
             return fail("dali_hip_lstm_recurrent_persistent: hs overlaps an input");
     }
     const int cus = compute_units();
@@ -552,7 +573,7 @@ extern "C" int dali_hip_lstm_recurrent_persistent(int steps, int batch, int hidd
         return fail("dali_hip_lstm_recurrent_persistent: an earlier persistent launch gave up waiting; call dali_hip_sync to collect that error first");
     if (!lds_kernel_serves(batch, hidden, cus)) {
         if ((size_t)batch * hidden * 4 >= 0x7ffffff0u) return fail("dali_hip_lstm_recurrent_persistent: state rows beyond the 2 GiB a buffer load addresses");
-        return lstm_recurrent_phased(steps, batch, hidden, pre, U, ldu, h0, c0, hs, c_out, g_status, cus);
+        return lstm_recurrent_phased(steps, batch, hidden, pre, bias, U, ldu, h0, c0, hs, c_out, g_status, cus);
     }
     // fewest hidden units per workgroup that still give every workgroup a compute unit of its own
     int HU = 1;
@@ -563,7 +584,7 @@ extern "C" int dali_hip_lstm_recurrent_persistent(int steps, int batch, int hidd
         return fail("dali_hip_lstm_recurrent_persistent: the slice of U per compute unit (%zu bytes) does not fit the LDS", lds_bytes);
     PersistentArgs a;
     a.T = steps; a.B = batch; a.H = hidden; a.HU = HU; a.ldu = ldu;
-    a.pre = pre; a.U = U; a.h0 = h0; a.c0 = c0; a.hs = hs; a.c_out = c_out;
+    a.pre = pre; a.bias = bias; a.U = U; a.h0 = h0; a.c0 = c0; a.hs = hs; a.c_out = c_out;
     // the last two counters of the workspace (zero at rest, like the reduction tickets)
     a.bar = (unsigned int*)workspace() + kWorkspaceCounters - 2;
     a.done = (unsigned int*)workspace() + kWorkspaceCounters - 1;

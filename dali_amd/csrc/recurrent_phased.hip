@@ -49,6 +49,7 @@ struct PhasedArgs {
     int T, B, H, HU, ldu, KQ;  // KQ = H / 64: trips of 16 values of k in a wave's quarter of the K range
     int PH;                    // phases: row blocks of 16 * MT rows that take turns
     const float* pre;          // [T, B, 4H] = x(t).W + b
+    const float* bias;         // [4H], added to pre (LSTM); may be null
     const float* U;            // [H, 4H], row stride ldu
     const float* h0;           // [B, H]
     const float* c0;           // [B, H]
@@ -189,7 +190,10 @@ __global__ __launch_bounds__(256) void lstm_phased_kernel(PhasedArgs a) {
             const int e = tid + 256 * i, rr = e / HU, row = r0 + rr, uu = e - rr * HU;
             const bool mine = rr < ROWS && row < B;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) pre4[i][g] = mine ? a.pre[((size_t)t * B + row) * 4 * H + (size_t)g * H + u0 + uu] : 0.0f;
+            for (int g = 0; g < 4; ++g) {
+                pre4[i][g] = mine ? a.pre[((size_t)t * B + row) * 4 * H + (size_t)g * H + u0 + uu] : 0.0f;
+                if (mine && a.bias) pre4[i][g] += a.bias[(size_t)g * H + u0 + uu];
+            }
         }
         f4 acc[MT][NT];
 #pragma unroll
@@ -395,7 +399,7 @@ int recurrent_phased_supported(int batch, int hidden, int cus) {
     return batch >= 1 && batch <= 128 && hidden >= 64 && hidden <= 2048 && hidden % 64 == 0 && units_per_workgroup(hidden, cus) != 0;
 }
 
-int lstm_recurrent_phased(int steps, int batch, int hidden, const float* pre, const float* U, int ldu, const float* h0, const float* c0, float* hs,
+int lstm_recurrent_phased(int steps, int batch, int hidden, const float* pre, const float* bias, const float* U, int ldu, const float* h0, const float* c0, float* hs,
                           float* c_out, int* status, int cus) {
     const int HU = units_per_workgroup(hidden, cus);
     if (!recurrent_phased_supported(batch, hidden, cus) || HU == 0)
@@ -403,7 +407,7 @@ int lstm_recurrent_phased(int steps, int batch, int hidden, const float* pre, co
                     "of 64 up to 2048)", batch, hidden, cus);
     PhasedArgs a = {};
     a.T = steps; a.B = batch; a.H = hidden; a.HU = HU; a.ldu = ldu; a.KQ = hidden / 64;
-    a.pre = pre; a.U = U; a.h0 = h0; a.c0 = c0; a.hs = hs; a.c_out = c_out;
+    a.pre = pre; a.bias = bias; a.U = U; a.h0 = h0; a.c0 = c0; a.hs = hs; a.c_out = c_out;
     a.status = status;
     static const unsigned int spin_env = getenv("DALI_HIP_PERSISTENT_SPIN_LIMIT") ? (unsigned int)atol(getenv("DALI_HIP_PERSISTENT_SPIN_LIMIT")) : (1u << 20);
     a.spin_limit = spin_env;
@@ -438,7 +442,7 @@ int gru_recurrent_phased(int steps, int batch, int hidden, const float* pre, con
                     "of 64 up to 2048)", batch, hidden, cus);
     PhasedArgs a = {};
     a.T = steps; a.B = batch; a.H = hidden; a.HU = HU; a.ldu = ldu; a.KQ = hidden / 64;
-    a.pre = pre; a.U = U; a.h0 = h0; a.hs = hs; a.rh = scratch;
+    a.pre = pre; a.bias = nullptr; a.U = U; a.h0 = h0; a.hs = hs; a.rh = scratch;
     a.status = status;
     static const unsigned int spin_env = getenv("DALI_HIP_PERSISTENT_SPIN_LIMIT") ? (unsigned int)atol(getenv("DALI_HIP_PERSISTENT_SPIN_LIMIT")) : (1u << 20);
     a.spin_limit = spin_env;

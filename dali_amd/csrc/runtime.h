@@ -81,7 +81,7 @@ hipError_t reserve_dynamic_lds(const void* kernel, size_t bytes);
 // 64 up to 2048 (weights in registers, two row blocks taking turns at the grid barrier). `status` is the host-visible word that a
 // workgroup sets when a wait gives up; `cus` the number of compute units of the bound device.
 int recurrent_phased_supported(int batch, int hidden, int cus);
-int lstm_recurrent_phased(int steps, int batch, int hidden, const float* pre, const float* U, int ldu, const float* h0, const float* c0, float* hs,
+int lstm_recurrent_phased(int steps, int batch, int hidden, const float* pre, const float* bias, const float* U, int ldu, const float* h0, const float* c0, float* hs,
                           float* c_out, int* status, int cus);
 int gru_recurrent_phased(int steps, int batch, int hidden, const float* pre, const float* U, int ldu, const float* h0, float* hs, float* scratch,
                          int* status, int cus);

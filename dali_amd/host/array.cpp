@@ -1705,11 +1705,11 @@ LSTMSequence lstm_sequence(const Array& xs, const Array& h0, const Array& c0, co
     // (a size that the persistent kernels do not serve, or serve more slowly than a launch per step, takes the loop below; a failure of the
     // launch itself is an error)
     if (persistent_ok) {
-        Array pre = add(dot(seq.reshape({T * Bn, In}), W), b.expand_dims(0));
+        Array pre = dot(seq.reshape({T * Bn, In}), W);
         pre.eval();
         Array c_last({Bn, H}, DTYPE_FLOAT);
         Array h0c = h0.offset() % 4 == 0 ? h0 : h0.ascontiguousarray();
-        lstm_recurrent_persistent(pre.reshape({T, Bn, 4 * H}), U, h0c, c0, hs, c_last);
+        lstm_recurrent_persistent(pre.reshape({T, Bn, 4 * H}), b, U, h0c, c0, hs, c_last);
         return {hs, c_last, hs[T - 1]};
     }
     Array c_prev = c0, h_prev = h0;

@@ -106,7 +106,7 @@ void lstm_step_fused(const Array& x, const Array& h, const Array& c, const Array
 void lstm_step_small(const Array& x, const Array& h, const Array& c, const Array& W, const Array& U, const Array& b, const Array& c_new,
                      const Array& h_new);
 // the recurrent half of an LSTM over a whole sequence in one launch: pre [T, B, 4H] = x.W + bias for every step
-void lstm_recurrent_persistent(const Array& pre, const Array& U, const Array& h0, const Array& c0, const Array& hs, const Array& c_out);
+void lstm_recurrent_persistent(const Array& pre, const Array& bias, const Array& U, const Array& h0, const Array& c0, const Array& hs, const Array& c_out);
 void gru_recurrent_persistent(const Array& pre, const Array& U, const Array& h0, const Array& hs, const Array& scratch);
 // softmax of a contiguous fp32 buffer seen as [outer, extent, inner] along `extent`, one pass over memory (records itself like any other launch)
 void softmax_axis_launch(const Array& x, const Array& out, long long outer, int extent, long long inner);
