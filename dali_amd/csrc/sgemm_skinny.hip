@@ -43,7 +43,10 @@ struct SkinnyArgs {
 // MT: 16-row tiles of A; G: trips of 16 values of k whose loads are issued together
 // TB: B is stored transposed, [N][K] with row length ldb (the weights of a layer kept as [outputs, inputs]). A lane then
 // loads four consecutive k of its column, as it does for its row of A, and a 16-column tile is 16 consecutive columns.
-template <int MT, int G, bool TB>
+// RAG: K is no multiple of 4 (the gradient of a layer's input over an odd vocabulary): what the last vector of a row brings from behind
+// K is set to zero in both operands. Such products went through the guarded tiles of 64 rows. us, before -> here: [3,15299].[15299,1024] with B stored
+// transposed 48 -> 14, [5,21678].[21678,2752] likewise 154 -> 54, [8,1001].[1001,1000] 17.4 -> 5.7, [32,165].[165,2304] 13.0 -> 5.8, [64,1001].[1001,32000] 100 -> 57.
+template <int MT, int G, bool TB, bool RAG>
 __global__ __launch_bounds__(256, 2) void sgemm_skinny_kernel(SkinnyArgs a) {
     extern __shared__ float red_flat[];  // [4 waves][4 column tiles][MT][16][16]
     float (*red)[4][MT][16][16] = reinterpret_cast<float (*)[4][MT][16][16]>(red_flat);
@@ -70,13 +73,13 @@ __global__ __launch_bounds__(256, 2) void sgemm_skinny_kernel(SkinnyArgs a) {
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             const int kk = kbase + 16 * (q0 + g) + 4 * kgrp;  // this lane's four values of k
-            const bool valid = q0 + g < trips && kk < K;      // (K is a multiple of 4: the four are inside or outside together)
+            const bool valid = q0 + g < trips && kk < K;      // (without RAG the four are inside or outside together)
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 // TB: c counts column tiles and the vector runs along k; otherwise c counts the lane's four rows of B and the
                 // vector runs along the columns
                 const int col = col0 + 16 * c + arow;
-                const int off = TB ? (col < N && valid ? (col * a.ldb + kk) * 4 : kOutside) : (valid ? (kk + c) * a.ldb * 4 + bcol : kOutside);
+                const int off = TB ? (col < N && valid ? (col * a.ldb + kk) * 4 : kOutside) : (valid && (!RAG || kk + c < K) ? (kk + c) * a.ldb * 4 + bcol : kOutside);
                 bv[g][c] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(brows, off, 0, 0));
             }
 #pragma unroll
@@ -84,6 +87,20 @@ __global__ __launch_bounds__(256, 2) void sgemm_skinny_kernel(SkinnyArgs a) {
                 const int row = 16 * m + arow;
                 av[g][m] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(arows, row < M && valid ? (row * a.lda + kk) * 4 : kOutside, 0, 0));
             }
+        }
+        if (RAG && kbase + 16 * (q0 + G) > K) {
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const bool behind = kbase + 16 * (q0 + g) + 4 * kgrp + j >= K;
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) av[g][m][j] = behind ? 0.0f : av[g][m][j];
+                    if (TB) {
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) bv[g][c][j] = behind ? 0.0f : bv[g][c][j];
+                    }
+                }
         }
 #pragma unroll
         for (int g = 0; g < G; ++g)
@@ -244,7 +261,7 @@ __global__ __launch_bounds__(256, 2) void sgemm_smallk_kernel(SmallKArgs a) {
 // 1: the product was launched; 0: not a case for this kernel (the caller takes the general path); -1: failure
 int sgemm_skinny(bool tb, int M, int N, int K, float alpha, const float* A, int lda, const float* B, int ldb, float beta, float* C, int ldc) {
     static const bool enabled = !(getenv("DALI_HIP_GEMM_SKINNY") && atoi(getenv("DALI_HIP_GEMM_SKINNY")) == 0);
-    if (!enabled || M < 1 || M > 64 || K < 64 || K % 4 != 0 || N < 64) return 0;
+    if (!enabled || M < 1 || M > 64 || K < 64 || N < 64) return 0;
     // 32-bit byte offsets into both operands
     if ((size_t)(tb ? N : K) * ldb * 4 + 4096 >= ((size_t)1 << 31) || (size_t)M * lda * 4 + 4096 >= ((size_t)1 << 31)) return 0;
     if (((uintptr_t)A | (uintptr_t)B) % 4 != 0) return 0;
@@ -260,7 +277,8 @@ int sgemm_skinny(bool tb, int M, int N, int K, float alpha, const float* A, int 
     if (blocks * KS < 32) return 0;
     // 33 to 64 rows with a split of K: the tiled kernel is as fast or faster unless the shares are long
     // (64 x 4096 over K = 1024: 16.4 against 22.9 us here; 64 x 1024 over K = 32000: 71 against 58 us)
-    if (KS > 1 && M > 32 && K / KS < (M > 48 ? 1536 : 1024)) return 0;
+    // (K off 4: the guarded tiles are slower, [64,3001].[3001,2000] 37 against 23 us, [33,15299].[15299,1024] 53 against 30)
+    if (K % 4 == 0 && KS > 1 && M > 32 && K / KS < (M > 48 ? 1536 : 1024)) return 0;
     if (KS > 1 && ((size_t)blocks * KS * M * kCols * sizeof(float) > kWorkspacePartialBytes || blocks > kWorkspaceCounters - 2)) KS = 1;
     SkinnyArgs a;
     a.M = M; a.N = N; a.K = K; a.KS = KS;
@@ -280,9 +298,11 @@ int sgemm_skinny(bool tb, int M, int N, int K, float alpha, const float* A, int 
         if (e == hipSuccess) hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds_bytes, stream(), a);
     };
     // (trips issued together: 1 to 8 measured alike, the compiler pipelines the loop; 4 is the best of them on short K shares)
-#define SKINNY_CASE(mt)                                           \
-    if (tb) launch(sgemm_skinny_kernel<mt, 4, true>);             \
-    else launch(sgemm_skinny_kernel<mt, 4, false>);               \
+#define SKINNY_CASE(mt)                                                     \
+    if (K % 4 == 0 && tb) launch(sgemm_skinny_kernel<mt, 4, true, false>);  \
+    else if (K % 4 == 0) launch(sgemm_skinny_kernel<mt, 4, false, false>);  \
+    else if (tb) launch(sgemm_skinny_kernel<mt, 4, true, true>);            \
+    else launch(sgemm_skinny_kernel<mt, 4, false, true>);                   \
     break;
     switch (MT) {
         case 1: SKINNY_CASE(1)
