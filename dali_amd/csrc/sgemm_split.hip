@@ -582,14 +582,16 @@ int choose_shares(const SplitArgs& g, int cus, double fp32_rate, bool long_rate,
     // 1.0; starting and ending a tile costs four slabs; adding shares up costs a launch and a read of them. The fp32 kernels by their
     // rate over whole 64x64 tiles, in TFLOP/s: 76 where several terms or a row map leave them the register-staged kernel (measured 68 to 94); 135
     // where their loads write LDS and up to four rounds of 64x64 tiles fill the chip (117 to 141); 115 over long inner extents, where they
-    // cut what does not fill a round into shares (117 to 136 at 1.4 to 2.4 tiles a compute unit); 112 else (45 to 145: operands off 16 bytes and rounds
-    // that are not full are the slow ones). Measured, us here / there, in the orders NN NT TN TT:
+    // cut what does not fill a round into shares (117 to 136 at 1.4 to 2.4 tiles a compute unit); 55 where operands lie off 16 bytes
+    // (22 to 81 over 64 products of odd sizes, of which the split form was the faster one in all above 10 us); 112 else (70 to 145: rounds that are not full are the slow ones). Measured, us here / there, in the orders NN NT TN TT:
     //   one 128x128 tile a compute unit, refused: 2048^2 over 512 39 38 40 38 / 37 36 35 36, over 1024 69 68 69 67 / 65 65 63 64; 1024^2 over 4096
     //     63 62 63 63 / 64 61 63 61; [1883,10136] against [4486,10136] (NT) 1485 / 1411; [256,4096] over 512 24 24 24 24 / 11 11 11 11
     //   two: [2048,4096] over 256 35 34 35 35 / 37 38 36 38, over 1024 107 105 106 106 / 124 126 122 125
     //   three: [3072,4096] over 256 52 51 52 51 / 53 54 53 54, over 1024 161 160 163 160 / 185 185 180 185, over 4096 605 599 612 598 / 711 713 698 713
     //   five: [4096,5120] over 256 79 78 80 79 / 87 88 85 87, over 1024 260 254 260 256 / 310 311 301 309
     //   2.4 tiles, off 16 bytes: [573,15415] over 2683 395 397 400 396 / 581 589 910 900
+    //   off 16 bytes: [1023,1025] over 1027 36 34 34 34 / 42 72 69 84, [172,60984] over 425 101 99 102 100 / 184 194 165 215, [999,1001] over 5001 81 81 78 81 / 179 146 206 251,
+    //     [2001,2003] over 301 31 30 31 30 / 72 62 54 56, [4099,515] over 259 27 25 27 26 / 32 53 36 43; refused: [700,701] over 703 24 24 24 24 / 26 33 27 33
     //   shares: [256,1024] over 32000 110 108 110 110 / 131 129 132 129; [576,128] over 93312 116 114 108 110 / 118 116 119 116
     //   rows of a convolution: [100352,128] over 3 x 192 122 / 166, [3136,256] over 3 x 384 30 / 27 (refused)
     const int most = (int)(kWorkspacePartialBytes / (kTile * kTile * sizeof(float)) / tiles);
@@ -662,7 +664,7 @@ int sgemm_split(bool ta, bool tb, int M, int N, int nseg, const int* K, const fl
     const long tiles64 = (long)((M + 63) / 64) * ((N + 63) / 64), rounds64 = (tiles64 + cus - 1) / cus;
     const bool fills = tiles <= cus && (double)tiles64 >= 0.95 * (double)(rounds64 * cus);
     const bool staged = nseg > 2 || map.on;
-    g.shares = choose_shares(g, cus, staged ? 76e6 : !direct ? 112e6 : fills ? 135e6 : 112e6, !staged && direct && !fills);
+    g.shares = choose_shares(g, cus, staged ? 76e6 : !direct ? 55e6 : fills ? 135e6 : 112e6, !staged && direct && !fills);
     if (g.shares == 0) return 0;
     if (!ta && !tb) return launch_split(g, sgemm_split_kernel<false, false, kPlain>);
     if (ta && !tb) return launch_split(g, sgemm_split_kernel<true, false, kPlain>);
