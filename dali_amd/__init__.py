@@ -1,4 +1,4 @@
-"""ctypes mirror of the C++ host front-end (``dali_amd/host/dali.h``).
+"""Scripting mirror of the C++ host front-end (``dali_amd/host/dali.h``).
 
 The package is a thin scripting binding: ``Array`` handles and the ``op``
 functions build the same lazy expressions a C++ user of the reference writes
