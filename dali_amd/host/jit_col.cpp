@@ -242,13 +242,14 @@ static std::string gen_col_kernel(const Program& P, int red_id, int dest_array, 
     auto emit_group_fold = [&](const std::string& ind) {
         ss << ind << "if (NWAVE > 1) {\n" << ind << "  _Pragma(\"unroll\") for (int j = 0; j < VEC; ++j) { sm[wave][lane * VEC + j] = acc[j];" << (ARG ? " smi[wave][lane * VEC + j] = acci[j];" : "")
            << " }\n" << ind << "  __syncthreads();\n";
-        ss << ind << "  if (threadIdx.x < TPP * VEC) {\n" << ind << "    " << t << " r = sm[0][threadIdx.x];\n";
+        // (strips of more than 256 columns, one or two row groups: several columns to a thread)
+        ss << ind << "  for (int c = threadIdx.x; c < TPP * VEC; c += 256) {\n" << ind << "    " << t << " r = sm[0][c];\n";
         if (ARG) {
-            ss << ind << "    int ri = smi[0][threadIdx.x];\n";
-            ss << ind << "    _Pragma(\"unroll\") for (int w = 1; w < NWAVE; ++w) { const " << t << " ov = sm[w][threadIdx.x]; const int oi = smi[w][threadIdx.x]; " << take("r", "ri", "ov", "oi") << " }\n";
-            ss << ind << "    sm[0][threadIdx.x] = r; smi[0][threadIdx.x] = ri;\n";
+            ss << ind << "    int ri = smi[0][c];\n";
+            ss << ind << "    _Pragma(\"unroll\") for (int w = 1; w < NWAVE; ++w) { const " << t << " ov = sm[w][c]; const int oi = smi[w][c]; " << take("r", "ri", "ov", "oi") << " }\n";
+            ss << ind << "    sm[0][c] = r; smi[0][c] = ri;\n";
         } else {
-            ss << ind << "    _Pragma(\"unroll\") for (int w = 1; w < NWAVE; ++w) r = " << red.name << "::step<" << t << ">(r, sm[w][threadIdx.x]);\n" << ind << "    sm[0][threadIdx.x] = r;\n";
+            ss << ind << "    _Pragma(\"unroll\") for (int w = 1; w < NWAVE; ++w) r = " << red.name << "::step<" << t << ">(r, sm[w][c]);\n" << ind << "    sm[0][c] = r;\n";
         }
         ss << ind << "  }\n" << ind << "  __syncthreads();\n" << ind << "  if (wave == 0) {\n" << ind << "    _Pragma(\"unroll\") for (int j = 0; j < VEC; ++j) { acc[j] = sm[0][lane * VEC + j];"
            << (ARG ? " acci[j] = smi[0][lane * VEC + j];" : "") << " }\n" << ind << "  }\n" << ind << "}\n";
@@ -423,7 +424,7 @@ bool try_col(const DestSpec& spec) {
     // slower: [3001,2047] 6.9 -> 8.2).
     int RG = streaming && size_of_dtype(arg.dtype()) == 4 ? 4 : 8;
     if (!streaming && (X <= 256 || (K >= 64 * max_blocks && X <= 1024))) RG = X > 64 ? 16 : (X <= 8 * 4 || K >= 64 * max_blocks ? 4 : 8);
-    if (rg_env > 0) RG = rg_env;
+    if (rg_env > 0 && 256 % rg_env == 0) RG = rg_env;  // (row groups of whole threads)
     // partial rows in flight in the fold (sixteen also leave the compiler the registers that exponentials in double precision want in
     // the main loop: sum(exp(x)) of [8192,8192] 110 us with eight, 97 with sixteen)
     const int TAIL = tail_env > 0 ? tail_env : (size_of_dtype(arg.dtype()) == 8 && contains_expensive(P, P.nodes[red_id].args[0]) ? 16 : 8);
