@@ -267,8 +267,9 @@ static std::string gen_col_kernel(const Program& P, int red_id, int dest_array, 
     ss << "  if (gridDim.y == 1) {\n    if (wave == 0 && k_ok) {\n";
     emit_store("      ");
     ss << "    }\n    return;\n  }\n";
-    // one counter a strip; a few strips with many workgroups each have groups of them (up to 16 behind the strip's own)
-    ss << "  const bool grouped = gridDim.x <= 15;\n";
+    // one counter a strip; a few strips with many workgroups each have groups of them (up to 16 behind the strip's own: from 1024 workgroups on
+    // dali_last_arrival takes 64, which would reach into the next strips')
+    ss << "  const bool grouped = gridDim.x <= 15 && gridDim.y < 1024;\n";
     ss << "  unsigned int* counters = (unsigned int*)A.ws + (grouped ? blockIdx.x * (17u * 64u) : blockIdx.x * dali_counter_step(gridDim.x));\n";
     ss << "  char* partials = (char*)A.ws + " << 16384 * 4 << ";\n";
     ss << "  const unsigned int KP = gridDim.x * TPP * VEC;  // padded kept extent of one row of partials\n";

@@ -33,6 +33,19 @@ def test_the_fold_takes_every_column_of_a_strip(D, groups, what):
     assert count == 1 or sorted(columns) == list(range(threads * vec))
 
 
+@pytest.mark.parametrize("strips", range(1, 17))
+def test_strips_draw_from_counters_of_their_own(D, strips):
+    text = run("D.generate_only([op.sum(D.Array.empty((5003, 300)), [0])])\nprint(D.last_source())")
+    body = text[text.rindex('extern "C" __global__'):]
+    grouped = re.search(r"const bool grouped = (.*);", body).group(1).replace("&&", "and").replace("gridDim.x", "strips").replace("gridDim.y", "blocks")
+    words = int(re.search(r"grouped \? blockIdx\.x \* \((\d+)u \* 64u\)", body).group(1)) * 64
+    line, below, above = (int(v) for v in re.search(r"groups = n < (\d+) \? (\d+) : (\d+);", text).groups())
+    for blocks in (2, 127, 128, 1023, 1024, 1025, 4096, 65535):
+        if eval(grouped, {"strips": strips, "blocks": blocks}):
+            groups = below if blocks < line else above
+            assert (1 + groups) * 64 <= words and strips * words <= 16384, (strips, blocks)
+
+
 WHOLE = """
 rng = np.random.RandomState(7)
 for rows, cols in ((1025, 3001), (64, 2048), (5003, 300), (33, 17), (3, 4100)):
@@ -50,3 +63,14 @@ for rows, cols in ((1025, 3001), (64, 2048), (5003, 300), (33, 17), (3, 4100)):
 @pytest.mark.parametrize("groups", ["1", "2", "4", "16", "64"])
 def test_row_groups(gpu, groups):
     run(WHOLE, DALI_HIP_COL_RG=groups)
+
+
+@pytest.mark.gpu
+def test_more_workgroups_to_a_strip_than_counters_in_its_groups(gpu):
+    run("""
+x = np.random.RandomState(3).randint(-8, 9, (40000, 300)).astype(np.float32)
+X = D.Array.from_numpy(x)
+for _ in range(3):
+    assert np.array_equal(op.sum(X, [0]).numpy(), x.sum(0)) and np.array_equal(op.argmax(X, 0).numpy(), x.argmax(0))
+    assert op.max(op.square(X)).numpy() == 64.0  # draws from the same counters
+""", DALI_HIP_COL_MAXY="2048", DALI_HIP_COL_BLOCKS="8192", DALI_HIP_COL_ROWS="8")
