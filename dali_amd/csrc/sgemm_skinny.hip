@@ -258,6 +258,25 @@ __global__ __launch_bounds__(256, 2) void sgemm_smallk_kernel(SmallKArgs a) {
 
 }  // namespace
 
+// Whether 33 to 48 rows (`wide`: 49 to 64) over a K off 4 are faster here than through the guarded tiles, which take 64 rows in the time of one. `direct`: the rows
+// of B start at 16-byte boundaries (the tiles are slowest there: they guard A and not B). From 384 column blocks on a product is not cut and always
+// faster here ([64,50257] over 129 30 us against 39); between 150 and 384 shares make more workgroups than fit the chip at once. Over 1600
+// products of 33 to 64 rows, 2050 to 32000 columns and K of 65 to 5001 this rule loses 7 % at most. us, tiles / here, taken:
+//   rows of B transposed: [64,8000] over 255 18.2 / 11.9, [64,2050] over 65 15.9 / 9.3, [64,2051] over 5001 48.2 / 50.5
+//   [48,4001] over 255 11.6 / 8.3, [40,10001] over 451 23.2 / 12.4, [40,10001] over 2001 87 / 46, [49,2050] over 201 11.5 / 8.7, [64,4001] over 1001 18.2 / 16.0
+//   direct: [64,3000] over 97 15.1 / 9.2, [64,8000] over 255 15.3 / 10.4
+// refused: [64,4001] over 97 7.5 / 9.2, over 351 10.6 / 14.7, [64,2050] over 3001 28.8 / 34.6, [64,16001] over 513 26.6 / 41.1, transposed 31.7 / 41.4,
+//   [48,4001] over 97 7.5 / 7.7, over 351 10.8 / 11.8, [48,24001] over 513 37 / 50, [56,12000] over 1501 39 / 58, [64,24001] over 65 10.8 / 14.2
+static bool ragged_pays(bool wide, bool tb, bool direct, int K, int KS, int blocks) {
+    if (blocks >= 384) return true;
+    if (blocks > 150 && KS > 1) return wide ? !direct && K >= 1500 && K / KS >= 500 : K / KS >= (direct ? 450 : 350);
+    if (tb) return true;
+    if (direct) return !wide || blocks <= 300 || K <= 256;
+    if (!wide) return K >= 128 && !(K > 320 && K < 513 && blocks <= 64) && !(K < 350 && blocks > 300);
+    if (blocks > 150) return blocks <= 300 && K >= 320;
+    return (K >= 192 && K <= 256) || (K >= 513 && K < 1200) || (K >= 2000 && blocks > 100);
+}
+
 // 1: the product was launched; 0: not a case for this kernel (the caller takes the general path); -1: failure
 int sgemm_skinny(bool tb, int M, int N, int K, float alpha, const float* A, int lda, const float* B, int ldb, float beta, float* C, int ldc) {
     static const bool enabled = !(getenv("DALI_HIP_GEMM_SKINNY") && atoi(getenv("DALI_HIP_GEMM_SKINNY")) == 0);
@@ -277,8 +296,8 @@ int sgemm_skinny(bool tb, int M, int N, int K, float alpha, const float* A, int 
     if (blocks * KS < 32) return 0;
     // 33 to 64 rows with a split of K: the tiled kernel is as fast or faster unless the shares are long
     // (64 x 4096 over K = 1024: 16.4 against 22.9 us here; 64 x 1024 over K = 32000: 71 against 58 us)
-    // (K off 4: the guarded tiles are slower, [64,3001].[3001,2000] 37 against 23 us, [33,15299].[15299,1024] 53 against 30)
     if (K % 4 == 0 && KS > 1 && M > 32 && K / KS < (M > 48 ? 1536 : 1024)) return 0;
+    if (K % 4 != 0 && M > 32 && !ragged_pays(M > 48, tb, !tb && ldb % 4 == 0, K, KS, blocks)) return 0;
     if (KS > 1 && ((size_t)blocks * KS * M * kCols * sizeof(float) > kWorkspacePartialBytes || blocks > kWorkspaceCounters - 2)) KS = 1;
     SkinnyArgs a;
     a.M = M; a.N = N; a.K = K; a.KS = KS;

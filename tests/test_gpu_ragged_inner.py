@@ -45,3 +45,11 @@ def test_at_most_64_rows(gpu, rng, M, N, K, tb):
             assert np.isnan(out[1, :N]).all()
         assert np.array_equal(out[rows, :N], want[rows])
         assert np.array_equal(out[:, N], c[:, N])
+
+
+# more than 32 rows: either side of the lines between the streamed form and the tiles (rows, column blocks, shares, alignment of the right operand's rows)
+@pytest.mark.parametrize("M,N", [(48, 4001), (49, 4001), (64, 4000), (33, 9601), (49, 9601), (48, 12000), (64, 12001), (49, 19265), (64, 24513)])
+@pytest.mark.parametrize("K", [97, 191, 201, 255, 257, 321, 451, 513, 701, 1201, 1501])
+@pytest.mark.parametrize("tb", [0, 1])
+def test_33_to_64_rows(gpu, rng, M, N, K, tb):
+    test_at_most_64_rows(gpu, rng, M, N, K, tb)
