@@ -423,12 +423,38 @@ bool try_col(const DestSpec& spec) {
     // [3001,2047] 12.0 -> 9.7, [8192,8192] 92 -> 87). Where a strip can be left to one workgroup, which then meets no others, as
     // many as its rows keep busy ([100,100] 4.0 -> 2.7, [256,32000] 5.1 -> 3.7, [64,65536] 2.7 with four, 2.9 with sixteen; sixteen with others to meet is
     // slower: [3001,2047] 6.9 -> 8.2).
-    int RG = streaming && size_of_dtype(arg.dtype()) == 4 ? 4 : 8;
+    // Much transcendental arithmetic on every element (`cost`: an exponential counts one, a longer function two, in double precision twice that): the
+    // rows that one thread takes in turn are then what a reduction of up to some hundred rows lasts, and waves with at most eight lanes at work (the
+    // last strip of a matrix, of few columns) take two to three times as long over a row. So from 144 rows on they are dealt out to more workgroups as
+    // long as the strips leave compute units idle, and no groups are taken that leave the last strip that thin where fewer do not. us, sum(x * tanh(y)) in
+    // double precision, without these lines / with: [256,1000] 24.9 / 15.8, [200,5000] 22.5 / 17.9, [256,48] 24.1 / 15.5, [256,900] 54 / 15.9, [5000,900] 102 / 52,
+    // [20000,900] 321 / 110; in 4-byte values, sigmoid, tanh and log together: [256,1000] 12.3 / 9.0, [257,900] 17.9 / 9.5. In double precision four groups also
+    // for some thousand columns and rows: [3000,6000] 107 / 98, [300,17000] 56 / 51.
+    const bool wide = size_of_dtype(arg.dtype()) == 8, heavy = contains_expensive(P, P.nodes[red_id].args[0]);
+    int cost = 0;
+    if (heavy) {
+        std::set<int> body;
+        body_nodes(P, P.nodes[red_id].args[0], body, true);
+        for (int id : body) {
+            const PNode& n = P.nodes[id];
+            if (n.kind == Kind::ELEMENTWISE && expensive_functor(n.name)) cost += (n.name == "functor::exp" ? 1 : 2) * (wide ? 2 : 1);
+        }
+    }
+    auto thin = [&](int rg) { return VEC == 4 && K > 1024 / rg && K % (1024 / rg) > 0 && K % (1024 / rg) * rg <= 128; };
+    int RG = streaming && !wide ? 4 : 8;
     if (!streaming && (X <= 256 || (K >= 64 * max_blocks && X <= 1024))) RG = X > 64 ? 16 : (X <= 8 * 4 || K >= 64 * max_blocks ? 4 : 8);
+    if (wide && cost && K >= 4000 && X > 256 && X < 4096) RG = 4;
+    if (cost > 2 && X >= 144 && X <= 256 && K < 8192) RG = K < 64 ? 16 : 4;
+    if (cost > 1 && thin(RG))
+        for (int rg = RG / 2; rg >= 4; rg /= 2)
+            if (!thin(rg)) {
+                RG = rg;
+                break;
+            }
     if (rg_env > 0 && 256 % rg_env == 0) RG = rg_env;  // (row groups of whole threads)
     // partial rows in flight in the fold (sixteen also leave the compiler the registers that exponentials in double precision want in
     // the main loop: sum(exp(x)) of [8192,8192] 110 us with eight, 97 with sixteen)
-    const int TAIL = tail_env > 0 ? tail_env : (size_of_dtype(arg.dtype()) == 8 && contains_expensive(P, P.nodes[red_id].args[0]) ? 16 : 8);
+    const int TAIL = tail_env > 0 ? tail_env : (wide && heavy ? 16 : 8);
     std::vector<Output> outs(1);
     outs[0].root = red_id;
     outs[0].array = dest_array;
@@ -457,7 +483,7 @@ bool try_col(const DestSpec& spec) {
         Kp->plan.work_count = 1;
         Kp->plan.work_per_block = (256 / RG) * VEC;
         Kp->plan.work2_begin = L.shape_pos[0] + 1;
-        Kp->plan.work2_per_block = rows_env > 0 ? rows_env : (RG == 16 ? 256 : UNR * RG);  // fewest reduced rows per y-block
+        Kp->plan.work2_per_block = rows_env > 0 ? rows_env : (RG == 16 && cost <= 2 ? 256 : UNR * RG);  // fewest reduced rows per y-block
         Kp->plan.max_blocks2 = maxy_env;
         Kp->plan.max_blocks = max_blocks;  // the y split fills what the column strips leave
         Kp->plan.ws_elsize = pair ? 8 : size_of_dtype(arg.dtype()) + (is_arg ? 4 : 0);  // a partial is a value, plus its index
