@@ -48,8 +48,8 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 struct PhasedArgs {
     int T, B, H, HU, ldu, KQ;  // KQ = H / 64: trips of 16 values of k in a wave's quarter of the K range
     int PH;                    // phases: row blocks of 16 * MT rows that take turns
-    const float* pre;          // [T, B, 4H] = x(t).W + b
-    const float* bias;         // [4H], added to pre (LSTM); may be null
+    const float* pre;          // LSTM: [T, B, 4H] = x(t).W; GRU: [T, B, 3H] = x(t).W + b
+    const float* bias;         // LSTM: [4H], added to pre; may be null
     const float* U;            // [H, 4H], row stride ldu
     const float* h0;           // [B, H]
     const float* c0;           // [B, H]
@@ -166,6 +166,11 @@ __global__ __launch_bounds__(256) void lstm_phased_kernel(PhasedArgs a) {
     float wreg[KQB][4][NT];
     load_weights<KQB, NT>(a.U, a.ldu, H, HU, 4, u0, KQ, kbase, arow, kgrp, 0, wreg);
     for (int e = tid; e < B * HU; e += 256) cells[e] = a.c0[(size_t)(e / HU) * H + u0 + e % HU];
+    // This workgroup's bias, gate by gate (without one -0, which leaves every value as it is). It is added where the gates are formed: added to the
+    // values of `pre` as they were fetched it made every gate's load wait for the one before (us, 32 steps: [64,640] 572 -> 514, [32,320] 339 -> 294,
+    // [96,1024] 967 -> 903, [32,2048] 808 -> 765).
+    __shared__ float biases[4 * 8];
+    if (tid < 4 * HU) biases[tid] = a.bias ? a.bias[(size_t)(tid / HU) * H + u0 + tid % HU] : -0.0f;
     if (tid == 0) give_up = 0;
     // the (row, hidden unit) pairs this thread finishes in a phase: pair e = tid + 256 i is row e / HU of the phase, unit e % HU
     constexpr int PP = (16 * MT * (NT * 4) + 255) / 256;
@@ -190,10 +195,7 @@ __global__ __launch_bounds__(256) void lstm_phased_kernel(PhasedArgs a) {
             const int e = tid + 256 * i, rr = e / HU, row = r0 + rr, uu = e - rr * HU;
             const bool mine = rr < ROWS && row < B;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                pre4[i][g] = mine ? a.pre[((size_t)t * B + row) * 4 * H + (size_t)g * H + u0 + uu] : 0.0f;
-                if (mine && a.bias) pre4[i][g] += a.bias[(size_t)g * H + u0 + uu];
-            }
+            for (int g = 0; g < 4; ++g) pre4[i][g] = mine ? a.pre[((size_t)t * B + row) * 4 * H + (size_t)g * H + u0 + uu] : 0.0f;
         }
         f4 acc[MT][NT];
 #pragma unroll
@@ -223,9 +225,9 @@ __global__ __launch_bounds__(256) void lstm_phased_kernel(PhasedArgs a) {
                     float s = 0.0f;
 #pragma unroll
                     for (int w = 0; w < 4; ++w) s += red[w][rr / 16][j / 16][(rr & 15) * 16 + (j & 15)];
-                    g4[g] = pre4[i][g] + s;
+                    g4[g] = (pre4[i][g] + biases[j]) + s;
                 }
-                const float zero[4] = {0.f, 0.f, 0.f, 0.f};  // the bias is part of `pre`
+                const float zero[4] = {0.f, 0.f, 0.f, 0.f};  // (the bias is in g4)
                 float cn, hn;
                 lstm_gates(g4[0], g4[1], g4[2], g4[3], zero, cells[row * HU + uu], &cn, &hn);
                 cells[row * HU + uu] = cn;

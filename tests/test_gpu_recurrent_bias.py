@@ -38,3 +38,9 @@ def test_bias_apart(gpu, rng, T, B, H):
     finally:
         for p in d.values():
             hip.dali_hip_free(p)
+
+
+# weights in registers: one and two 16-column tiles, one and two row tiles to a turn, one to eight turns, the last one partly filled
+@pytest.mark.parametrize("T,B,H", [(3, 8, 640), (4, 64, 640), (3, 17, 320), (3, 32, 2048), (3, 33, 1536), (2, 128, 1024), (2, 100, 64), (3, 1, 1920)])
+def test_bias_apart_with_weights_in_registers(gpu, rng, T, B, H):
+    test_bias_apart(gpu, rng, T, B, H)
