@@ -73,6 +73,7 @@ int sgemm_split(bool ta, bool tb, int M, int N, int nseg, const int* K, const fl
                 float beta, float* C, int ldc, const SgemmRowMap& map, int cus);
 int split_conv_nhwc(bool filters_gradient, int n, int h, int w, int c, int f, int fh, int fw, int stride_h, int stride_w, const float* image, const float* other,
                     float* result, int cus);
+bool split_conv_nhwc_takes(bool filters_gradient, int n, int h, int w, int c, int f, int fh, int fw, int stride_h, int stride_w, int cus);
 // hipFuncSetAttribute(MaxDynamicSharedMemorySize) once per kernel: later launches of that kernel, which may be recorded into a
 // graph, are launches only. Keyed on the kernel's address (kernels of one signature share a function type, so a flag inside a
 // generic lambda or template would be shared among them).

@@ -1238,6 +1238,12 @@ int dali_hip_sgemm_terms(int nterms, int transA, int transB, int M, int N, const
     return sgemm_rowmajor(nterms, transA != 0, transB != 0, M, N, K, A, ldas, B, ldbs, alpha, beta, C, ldc, true, row_map);
 }
 
+int dali_hip_conv2d_nhwc_supported(int filters_gradient, int batch, int in_h, int in_w, int channels, int filters, int filter_h, int filter_w, int stride_h, int stride_w) {
+    if (ensure_init()) return 0;
+    if (batch < 1 || in_h < 1 || in_w < 1 || channels < 1 || filters < 1 || filter_h < 1 || filter_w < 1 || stride_h < 1 || stride_w < 1) return 0;
+    return split_conv_nhwc_takes(filters_gradient != 0, batch, in_h, in_w, channels, filters, filter_h, filter_w, stride_h, stride_w, device_cus());
+}
+
 int dali_hip_conv2d_nhwc(int filters_gradient, int batch, int in_h, int in_w, int channels, int filters, int filter_h, int filter_w, int stride_h, int stride_w,
                          const float* image, const float* other, float* result, int* taken) {
     if (ensure_init()) return DALI_HIP_ERROR;

@@ -672,18 +672,13 @@ int sgemm_split(bool ta, bool tb, int M, int N, int nseg, const int* K, const fl
     return launch_split(g, sgemm_split_kernel<true, true, kPlain>);
 }
 
-// The convolution of a channels-last image [n, h, w, c] with filters [f, fh, fw, c], without padding, and the gradient of its filters, as products whose
-// one operand is the image itself, read window by window: no patch matrix is written or read, and no padded copy of the image. `result`
-// as the matrix product lays it out: [n, out_h, out_w, f] (filters_gradient: [f, fh, fw, c], from `out` [n, out_h, out_w, f]). Taken where the rule above takes
-// the product of that size. 1: launched; 0: not a case for it (form the patch matrix); -1: failure (message set).
-// What the product alone takes is left: us, image padded or patch matrix formed first / here, [32,56,56,64] with 128 filters of 3x3 147 / 107 and gradient 169 / 112, at stride
-// 2 58 / 45 and 67 / 45; [8,64,64,33], 100 of 5x5 120 / 65 and 216 / 59; [32,56,56,128], 128 of 3x3 248 / 190 and 280 / 180; [64,28,28,256], 256 of 1x1 95 / 65 and 75 / 64.
-int split_conv_nhwc(bool filters_gradient, int n, int h, int w, int c, int f, int fh, int fw, int stride_h, int stride_w, const float* image, const float* other,
-                    float* result, int cus) {
+// What a convolution reads and how it is cut, all but the operands' addresses; false: not a case for it. (A function of the extents alone, so that it can be asked
+// before operands are laid out and a result is allocated.)
+static bool plan_conv_nhwc(SplitArgs& g, bool filters_gradient, int n, int h, int w, int c, int f, int fh, int fw, int stride_h, int stride_w, int cus) {
     const int oh = (h - fh) / stride_h + 1, ow = (w - fw) / stride_w + 1;
     const long positions = (long)n * oh * ow, run = (long)fw * c;
-    if (!split_enabled(cus) || h < fh || w < fw || (long)n * h * w * c >= (1L << 30) || positions * f >= (1L << 30) || (long)f * fh * run >= (1L << 30)) return 0;
-    SplitArgs g = {};
+    if (!split_enabled(cus) || h < fh || w < fw || (long)n * h * w * c >= (1L << 30) || positions * f >= (1L << 30) || (long)f * fh * run >= (1L << 30)) return false;
+    g = {};
     SplitConv& cv = g.cv;
     cv.out_w = ow;
     cv.out_h = oh;
@@ -704,39 +699,56 @@ int split_conv_nhwc(bool filters_gradient, int n, int h, int w, int c, int f, in
     divide_by((unsigned)run, &cv.run_m, &cv.run_s);
     if (filters_gradient) {
         g.nseg = 1;
-        g.A[0] = other;
         g.lda[0] = f;
-        g.B[0] = image;
         g.K[0] = (int)positions;
         g.M = f;
         g.N = fh * (int)run;
     } else {
-        if (fh > kMaxTerms) return 0;
+        if (fh > kMaxTerms) return false;
         g.nseg = fh;
         for (int s = 0; s < fh; ++s) {
-            g.A[s] = image + (size_t)s * cv.line;
-            g.B[s] = other + (size_t)s * run;
             g.ldb[s] = fh * (int)run;
             g.K[s] = (int)run;
         }
         g.M = (int)positions;
         g.N = f;
     }
-    if (g.M <= 64 || g.N <= 64 || g.K[0] <= 64) return 0;
+    if (g.M <= 64 || g.N <= 64 || g.K[0] <= 64) return false;
     for (int s = 0; s < g.nseg; ++s) g.slabs += (g.K[s] + kSlab - 1) / kSlab;
-    g.C = result;
     g.ldc = g.N;
     g.alpha = 1.0f;
     g.tiles_m = (g.M + kTile - 1) / kTile;
     g.tiles_n = (g.N + kTile - 1) / kTile;
-    if ((long)g.tiles_m * g.tiles_n > (1L << 24)) return 0;
+    if ((long)g.tiles_m * g.tiles_n > (1L << 24)) return false;
     // what it stands in for: a launch that forms a patch matrix, written and read at about 4.5 TB/s, and a product (off 16 bytes at 40 to 60 TFLOP/s); at stride 1 and
     // whole vectors of channels a padded copy of the image and a sum of products
     const double product = c % 4 == 0 && f % 4 == 0 ? 112e6 : 60e6, patches = 5.0 + 8.0 * (double)positions * (fh * run) / 4.5e6;
     const bool summed = !filters_gradient && stride_h == 1 && stride_w == 1 && c % 4 == 0;
     g.shares = choose_shares(g, cus, summed ? 76e6 : product, false, summed ? 5.0 + 8.0 * n * h * w * c / 4.5e6 : patches);
-    if (g.shares == 0) return 0;
+    return g.shares != 0;
+}
+
+// The convolution of a channels-last image [n, h, w, c] with filters [f, fh, fw, c], without padding, and the gradient of its filters, as products whose
+// one operand is the image itself, read window by window: no patch matrix is written or read, and no padded copy of the image. `result`
+// as the matrix product lays it out: [n, out_h, out_w, f] (filters_gradient: [f, fh, fw, c], from `out` [n, out_h, out_w, f]). Taken where the rule above takes
+// the product of that size. 1: launched; 0: not a case for it (form the patch matrix); -1: failure (message set).
+// What the product alone takes is left: us, image padded or patch matrix formed first / here, [32,56,56,64] with 128 filters of 3x3 147 / 107 and gradient 169 / 112, at stride
+// 2 58 / 45 and 67 / 45; [8,64,64,33], 100 of 5x5 120 / 65 and 216 / 59; [32,56,56,128], 128 of 3x3 248 / 190 and 280 / 180; [64,28,28,256], 256 of 1x1 95 / 65 and 75 / 64.
+int split_conv_nhwc(bool filters_gradient, int n, int h, int w, int c, int f, int fh, int fw, int stride_h, int stride_w, const float* image, const float* other,
+                    float* result, int cus) {
+    SplitArgs g;
+    if (!plan_conv_nhwc(g, filters_gradient, n, h, w, c, f, fh, fw, stride_h, stride_w, cus)) return 0;
+    for (int s = 0; s < g.nseg; ++s) {
+        g.A[s] = filters_gradient ? other : image + (size_t)s * g.cv.line;
+        g.B[s] = filters_gradient ? image : other + (size_t)s * g.cv.run;
+    }
+    g.C = result;
     return launch_split(g, filters_gradient ? sgemm_split_kernel<true, false, kFilters> : sgemm_split_kernel<false, true, kWindows>);
+}
+
+bool split_conv_nhwc_takes(bool filters_gradient, int n, int h, int w, int c, int f, int fh, int fw, int stride_h, int stride_w, int cus) {
+    SplitArgs g;
+    return plan_conv_nhwc(g, filters_gradient, n, h, w, c, f, fh, fw, stride_h, stride_w, cus);
 }
 
 }  // namespace dali_hip

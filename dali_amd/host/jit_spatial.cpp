@@ -488,11 +488,12 @@ static Array conv2d_nhwc_direct(const Array& x_in, const Array& filters_in, int 
 }
 
 // The convolution of a channels-last image without padding, or the gradient of its filters, read from the image window by window
-// (dali_hip_conv2d_nhwc). False where the library does not take the size.
+// (dali_hip_conv2d_nhwc). False where the library does not take the size; then nothing has been evaluated, copied or allocated.
 static bool conv2d_nhwc_by_windows(bool filters_gradient, const Array& image_in, const Array& other_in, const std::vector<int>& result_shape, int f, int fh, int fw, int stride_h,
                                    int stride_w, Array* result) {
+    const std::vector<int> s = image_in.shape();
+    if (!dali_hip_conv2d_nhwc_supported(filters_gradient, s[0], s[1], s[2], s[3], f, fh, fw, stride_h, stride_w)) return false;
     Array image = dense_buffer(image_in), other = dense_buffer(other_in);
-    const std::vector<int> s = image.shape();
     Array out(result_shape, DTYPE_FLOAT);
     const float* ip = (const float*)image.device_ptr();
     const float* op_ = (const float*)other.device_ptr();
@@ -500,9 +501,9 @@ static bool conv2d_nhwc_by_windows(bool filters_gradient, const Array& image_in,
     auto issue = [=]() {
         int taken = 0;
         check_hip(dali_hip_conv2d_nhwc(filters_gradient, s[0], s[1], s[2], s[3], f, fh, fw, stride_h, stride_w, ip, op_, rp, &taken), "convolution product");
-        return taken != 0;
+        DALI_ASSERT(taken != 0, "internal: a convolution that the library said it takes was refused");
     };
-    if (!issue()) return false;
+    issue();
     jit_stats().gemms_launched++;
     if (g_recording) {
         note_recorded_write(out.expression()->memory);

@@ -256,6 +256,9 @@ int dali_hip_sgemm_terms(int nterms, int transA, int transB, int M, int N, const
  * Replaces im2col + op::dot (dali/array/op/conv.cpp:253-272, 369-392) for NHWC. */
 int dali_hip_conv2d_nhwc(int filters_gradient, int batch, int in_h, int in_w, int channels, int filters, int filter_h, int filter_w, int stride_h, int stride_w,
                          const float* image, const float* other, float* result, int* taken);
+/* Whether dali_hip_conv2d_nhwc takes these extents on the bound device (it asks nothing else of its operands): 1 yes, 0 no. No error is set. */
+int dali_hip_conv2d_nhwc_supported(int filters_gradient, int batch, int in_h, int in_w, int channels, int filters, int filter_h, int filter_w, int stride_h,
+                                   int stride_w);
 
 /*
  * One LSTM cell step in a single launch: pre = X[batch, input] . W[input, 4 hidden] + Hprev[batch, hidden] .

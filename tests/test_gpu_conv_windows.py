@@ -79,3 +79,25 @@ def test_a_recording_reads_what_its_operands_hold(gpu, D, rng):
             X.assign(D.Array.from_numpy(x))
             recording.replay(1)
             assert np.array_equal(y.numpy().reshape(-1, 128), windows64(x, (3, 3), (1, 1))[1] @ k.reshape(128, -1).T.astype(np.float64))
+
+
+# 64 filters: more than 1e9 operations, but a size that the products by windows do not take
+def test_a_size_that_is_not_taken_has_its_image_copied_once(gpu, D, rng):
+    n, h, w, c, f = 28, 44, 40, 40, 64
+    wide = rng.randint(-4, 5, (n, h, w, c + 1)).astype(np.float32)
+    x, k = np.ascontiguousarray(wide[..., 1:]), rng.randint(-4, 5, (f, 3, 3, c)).astype(np.float32)
+    dy = rng.randint(-4, 5, (n, h - 2, w - 2, f)).astype(np.float32)
+    for gradient in (0, 1):
+        assert gpu.dali_hip_conv2d_nhwc_supported(gradient, n, h, w, c, f, 3, 3, 1, 1) == 0 and gpu.dali_hip_conv2d_nhwc_supported(gradient, n, h, w, c, 2 * f, 3, 3, 1, 1) == 1
+    K, dY = D.Array.from_numpy(k), D.Array.from_numpy(dy)
+    _, patches = windows64(x, (3, 3), (1, 1))
+    launches = []
+    for X in (D.Array.from_numpy(x), D.Array.from_numpy(wide)[:, :, :, 1:]):
+        with D.Recording() as forward:
+            y = D.op.conv2d(X, K, 1, 1, "valid", "NHWC").eval()
+        with D.Recording() as backward:
+            dk = D.op.conv2d_backward_filters(X, dY, 1, 1, k.shape, "valid", "NHWC").eval()
+        launches.append((forward.launches, backward.launches))
+        assert np.array_equal(y.numpy().reshape(-1, f), patches @ k.reshape(f, -1).T)
+        assert np.array_equal(dk.numpy().reshape(f, -1), dy.reshape(-1, f).T @ patches)
+    assert launches[1] == (launches[0][0] + 1, launches[0][1] + 1), launches
