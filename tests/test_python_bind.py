@@ -83,3 +83,24 @@ def test_threads_build_and_generate(D):
     for t in threads:
         t.join()
     assert not failures
+
+
+def test_the_release_of_a_buffer_lets_other_threads_run(D):
+    x = D.Array.from_numpy(np.ones(1 << 26, np.float32))  # 256 MiB on the host: giving them back takes milliseconds
+    go, ran = threading.Event(), []
+
+    def other():
+        go.wait()
+        ran.append(True)
+    thread = threading.Thread(target=other)
+    thread.start()
+    interval = sys.getswitchinterval()
+    sys.setswitchinterval(60.0)  # nobody is made to give up the interpreter lock
+    try:
+        go.set()
+        del x
+        seen = bool(ran)
+    finally:
+        sys.setswitchinterval(interval)
+        thread.join()
+    assert seen
