@@ -160,6 +160,17 @@ PyObject* get_handle(PyObject* self, void*) {
     return PyLong_FromVoidPtr(of(self));
 }
 
+// (the handle is exchanged, not released: whoever assigns None has taken it over)
+int set_handle(PyObject* self, PyObject* value, void*) {
+    void* h = nullptr;
+    if (value && value != Py_None) {
+        h = PyLong_AsVoidPtr(value);
+        if (!h && PyErr_Occurred()) return -1;
+    }
+    ((ArrayObject*)self)->handle = h;
+    return 0;
+}
+
 PyObject* extents(PyObject* self, int (*read)(dali_array_t, int*), const char* what) {
     const int nd = dali_fe_ndim(of(self));
     if (nd < 0) return fail(what);
@@ -214,7 +225,7 @@ PyObject* nb_negative(PyObject* a) {
     return r.set(a) ? wrap(unlocked([&] { return dali_fe_binary("eltmul", l.handle, r.handle); }), "eltmul") : nullptr;
 }
 
-PyGetSetDef handle_getset[] = {{"_h", get_handle, nullptr, "the native handle", nullptr},
+PyGetSetDef handle_getset[] = {{"_h", get_handle, set_handle, "the native handle", nullptr},
                                {"shape", get_shape, nullptr, nullptr, nullptr},
                                {"strides", get_strides, nullptr, nullptr, nullptr},
                                {"ndim", get_ndim, nullptr, nullptr, nullptr},

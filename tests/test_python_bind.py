@@ -104,3 +104,15 @@ def test_the_release_of_a_buffer_lets_other_threads_run(D):
         sys.setswitchinterval(interval)
         thread.join()
     assert seen
+
+
+def test_the_handle_can_be_taken_over(D):
+    x = D.Array.from_numpy(np.arange(6, dtype=np.float32))
+    handle, x._h = x._h, None
+    assert x._h is None
+    y = D.Array(handle)
+    del x  # released nothing
+    assert y.shape == (6,) and np.array_equal(y.numpy(), np.arange(6, dtype=np.float32))
+    with pytest.raises(TypeError):
+        y._h = "text"
+    assert y._h == handle
