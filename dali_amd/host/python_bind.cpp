@@ -121,12 +121,12 @@ bool whole_numbers(PyObject* o, std::vector<int>* out) {
         out->resize(1);
         return whole_number(o, out->data());
     }
-    PyObject* s = PySequence_Fast(o, "expected a sequence of whole numbers");
+    PyObject* s = PySequence_Tuple(o);  // (converting an entry may run the program's code, which could change a list)
     if (!s) return false;
-    const Py_ssize_t n = PySequence_Fast_GET_SIZE(s);
+    const Py_ssize_t n = PyTuple_GET_SIZE(s);
     out->resize(n);
     bool ok = true;
-    for (Py_ssize_t i = 0; ok && i < n; ++i) ok = whole_number(PySequence_Fast_GET_ITEM(s, i), &(*out)[i]);
+    for (Py_ssize_t i = 0; ok && i < n; ++i) ok = whole_number(PyTuple_GET_ITEM(s, i), &(*out)[i]);
     Py_DECREF(s);
     return ok;
 }

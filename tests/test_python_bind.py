@@ -116,3 +116,18 @@ def test_the_handle_can_be_taken_over(D):
     with pytest.raises(TypeError):
         y._h = "text"
     assert y._h == handle
+
+
+def test_axes_that_change_their_list_when_they_are_read(D):
+    x, axes = D.Array.empty((4, 5, 6)), []
+
+    class Axis(object):
+        def __int__(self):
+            axes.clear()
+            return 0
+
+        __index__ = __int__
+    axes.extend([Axis(), 1, 2])
+    assert D.op.sum(x, axes).shape == ()  # the three that were given
+    axes.extend([Axis(), 2, 1])
+    assert x.transpose(axes).shape == (4, 6, 5)
