@@ -30,7 +30,7 @@ hip, front = _load()
 try:
     from . import _bind  # noqa: F401  (built on libdali_front)
 except ImportError as e:
-    raise ImportError("native library dali_amd/_bind.so is missing or does not load (%s): build it with `python -c 'import __graft_entry__ as g; g.build()'` "
+    raise ImportError("native library dali_amd/_bind is missing for this interpreter or does not load (%s): build it with `python -c 'import __graft_entry__ as g; g.build()'` "
                       "from the repository root (there is no fallback path)" % e)
 
 H = C.c_void_p

@@ -2,6 +2,7 @@
 import ctypes
 import gc
 import sys
+import sysconfig
 import threading
 
 import numpy as np
@@ -131,3 +132,8 @@ def test_axes_that_change_their_list_when_they_are_read(D):
     assert D.op.sum(x, axes).shape == ()  # the three that were given
     axes.extend([Axis(), 2, 1])
     assert x.transpose(axes).shape == (4, 6, 5)
+
+
+def test_the_extension_is_named_for_this_interpreter(D):
+    suffix = sysconfig.get_config_var("EXT_SUFFIX")
+    assert D._native._bind.__file__.endswith("_bind" + suffix) and suffix != ".so"
