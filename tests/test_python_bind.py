@@ -67,7 +67,7 @@ def test_operands_live_as_long_as_what_is_built_on_them(D):
     assert isinstance(y._h, int) and y._h != (y + 0)._h
 
 
-def test_threads_build_and_generate(D):
+def test_threads_build_nodes(D):
     failures = []
 
     def work(k):
