@@ -138,6 +138,7 @@ FRONT_SYMBOLS = {
     "dali_fe_scalar_int": (H, [_i]),
     "dali_fe_clone_handle": (H, [H]),
     "dali_fe_release": (None, [H]),
+    "dali_fe_is_last_handle": (_i, [H]),
     "dali_fe_ndim": (_i, [H]),
     "dali_fe_shape": (_i, [H, _ip]),
     "dali_fe_dtype": (_i, [H]),

@@ -57,6 +57,7 @@ dali_array_t dali_fe_scalar_float(float v) { FE_TRY(return wrap(Array(v));, null
 dali_array_t dali_fe_scalar_int(int v) { FE_TRY(return wrap(Array(v));, nullptr) }
 dali_array_t dali_fe_clone_handle(dali_array_t a) { FE_TRY(return wrap(A(a));, nullptr) }
 void dali_fe_release(dali_array_t a) { delete (Array*)a; }
+int dali_fe_is_last_handle(dali_array_t a) { FE_TRY(return A(a).state_.use_count() == 1 ? 1 : 0;, -1) }
 
 int dali_fe_ndim(dali_array_t a) { FE_TRY(return A(a).ndim();, -1) }
 int dali_fe_shape(dali_array_t a, int* out) {

@@ -4,8 +4,9 @@
 // and 0.8 to 2 us a node where this takes 0.1 to 0.3 (an expression of eight operators: 11.3 us to build, now 2.9; with its evaluation 16.8, now 8.3).
 //
 // Calls on operands give up the interpreter lock, as ctypes does: building a node may evaluate what it stands on, and observers of that may be
-// Python functions of another thread. So does the release of a buffer, which waits for transfers that still use its memory. Inspection, literals and
-// the release of nodes that were not evaluated keep it (giving it up costs 0.04 us).
+// Python functions of another thread. So does the release of the last handle to a buffer, or to a node that may hold the last reference to one: it
+// waits for transfers that still use the memory. Inspection, literals and the release of operands that a node keeps alive hold it (giving
+// it up costs 0.04 us).
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -36,7 +37,7 @@ auto unlocked(F&& call) {
 }
 
 void release(dali_array_t handle) {
-    if (dali_fe_is_buffer(handle)) {
+    if (dali_fe_is_last_handle(handle)) {
         unlocked([&] {
             dali_fe_release(handle);
             return 0;

@@ -34,6 +34,8 @@ dali_array_t dali_fe_scalar_float(float v);
 dali_array_t dali_fe_scalar_int(int v);
 dali_array_t dali_fe_clone_handle(dali_array_t a);
 void dali_fe_release(dali_array_t a);
+/* 1 where nothing else refers to what the handle stands for: releasing it gives that back, with buffers that nothing else uses */
+int dali_fe_is_last_handle(dali_array_t a);
 
 /* inspection */
 int dali_fe_ndim(dali_array_t a);

@@ -86,8 +86,11 @@ def test_threads_build_nodes(D):
     assert not failures
 
 
-def test_the_release_of_a_buffer_lets_other_threads_run(D):
+@pytest.mark.parametrize("what", ["buffer", "node that holds the last reference to one"])
+def test_the_release_of_a_buffer_lets_other_threads_run(D, what):
     x = D.Array.from_numpy(np.ones(1 << 26, np.float32))  # 256 MiB on the host: giving them back takes milliseconds
+    if what != "buffer":
+        x = x * 2.0
     go, ran = threading.Event(), []
 
     def other():
