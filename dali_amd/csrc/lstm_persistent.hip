@@ -10,8 +10,8 @@
 //   1. multiplies the previous hidden state h(t-1) [B, H] (read from global memory: it is the only thing the
 //      workgroups exchange) with its slice of U on the matrix cores (v_mfma_f32_16x16x4_f32, the K range split over
 //      the four waves and folded through LDS),
-//   2. adds the input half of the pre-activations, pre[t] = x(t).W + bias, which does not depend on h and is computed
-//      for all steps at once by one large product before this kernel runs,
+//   2. adds the input half of the pre-activations, pre[t] = x(t).W, which does not depend on h and is computed for all
+//      steps at once by one large product before this kernel runs, and the bias (unless pre holds it),
 //   3. applies the gates for its hidden units (same arithmetic, operation by operation, as the fused single step:
 //      double-precision sigmoid, tanhf, no contraction) and writes its HU columns of h(t),
 //   4. meets the other workgroups at a barrier (a counter in global memory) so that h(t) is complete before anyone
@@ -151,14 +151,18 @@ __global__ __launch_bounds__(256) void lstm_persistent_kernel(PersistentArgs a) 
     // so the step needs no cache-wide release or acquire: those fences write back and invalidate the whole second-level
     // cache and took 15 to 24 us of a step.
     float pre4[4] = {0.f, 0.f, 0.f, 0.f};
+    // The bias of this thread's gates (-0 leaves every value as it is), added as `pre` is fetched: the wave has those values before it begins to wait for
+    // h. Added where the gates are formed, so that the loads are in flight while h is waited for, it made a step slower: 8 rows of 1024 4.5 -> 5.1 us, 32 rows
+    // 8.3 -> 9.0, 64 rows 13.3 -> 13.6, 8 rows of 256 2.8 -> 3.7.
+    float bias4[4] = {-0.f, -0.f, -0.f, -0.f};
+    if (owner && a.bias) {
+#pragma unroll
+        for (int gate = 0; gate < 4; ++gate) bias4[gate] = a.bias[(size_t)gate * H + u0 + puu];
+    }
     auto fetch_pre = [&](int t) {
         if (owner) {
 #pragma unroll
-            for (int gate = 0; gate < 4; ++gate) pre4[gate] = a.pre[((size_t)t * B + pb) * 4 * H + (size_t)gate * H + u0 + puu];
-            if (a.bias) {
-#pragma unroll
-                for (int gate = 0; gate < 4; ++gate) pre4[gate] += a.bias[(size_t)gate * H + u0 + puu];
-            }
+            for (int gate = 0; gate < 4; ++gate) pre4[gate] = a.pre[((size_t)t * B + pb) * 4 * H + (size_t)gate * H + u0 + puu] + bias4[gate];
         }
     };
     fetch_pre(0);
@@ -306,7 +310,7 @@ __global__ __launch_bounds__(256) void lstm_persistent_kernel(PersistentArgs a) 
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();  // (also: the fold area is free again)
         if (tid == 0) __hip_atomic_fetch_add(a.bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        fetch_pre(t + 1);  // does not depend on h: in flight during the wait
+        fetch_pre(t + 1);  // does not depend on h: fetched while the others arrive
         if (tid == 0 && !wait_for(gridDim.x * (unsigned int)(t + 1))) give_up = 1;
         __syncthreads();
     }
@@ -524,7 +528,7 @@ static int compute_units() {
 }
 
 // the kernel that keeps U in LDS: up to 64 rows of 256, 512, 768 or 1024 hidden units (faster than the phased kernel wherever it
-// runs: 19 against 21 us per step at 64 rows of 1024, 12 against 13.4 at 32)
+// runs, us per step: 13.3 against 15.7 at 64 rows of 1024, 8.2 against 10.0 at 32; the nearest is 10.7 against 11.7 at 64 rows of 256)
 static bool lds_kernel_serves(int batch, int hidden, int cus) {
     // DALI_HIP_PERSISTENT_PHASED=1: never this kernel (for comparisons and tests of the other)
     static const bool phased_only = getenv("DALI_HIP_PERSISTENT_PHASED") && atoi(getenv("DALI_HIP_PERSISTENT_PHASED")) == 1;
@@ -599,7 +603,7 @@ extern "C" int dali_hip_lstm_recurrent_persistent_bias(int steps, int batch, int
     const int KQ = hidden / 64;
     // Waiting on the values themselves beats the barrier up to 32 rows (3.7 / 4.9 / 8.8 us a step at 1 / 8 / 32 rows of
     // 1024 units against 6.6 / 7.5 / 10.3); from 33 rows on the tiles that have to be fetched a second time cost more than
-    // the barrier (12.8 against 11.3 us at 33 rows, 17.4 against 13.6 at 64). DALI_HIP_PERSISTENT_DATA_FLAGS=0: always barriers.
+    // the barrier (before the weights were in registers 12.8 against 11.3 us at 33 rows, 17.4 against 13.6 at 64). DALI_HIP_PERSISTENT_DATA_FLAGS=0: always barriers.
     static const bool flags_allowed = !(getenv("DALI_HIP_PERSISTENT_DATA_FLAGS") && atoi(getenv("DALI_HIP_PERSISTENT_DATA_FLAGS")) == 0);
     const bool data_flags = flags_allowed && MT <= 2;
 #define DALI_PERSISTENT_CASE(mt, kq)                                              \
