@@ -105,15 +105,19 @@ void lstm_step_fused(const Array& x, const Array& h, const Array& c, const Array
                      const Array& h_new);
 void lstm_step_small(const Array& x, const Array& h, const Array& c, const Array& W, const Array& U, const Array& b, const Array& c_new,
                      const Array& h_new);
-// the recurrent half of an LSTM over a whole sequence in one launch: pre [T, B, 4H] = x.W + bias for every step
+// the recurrent half of an LSTM over a whole sequence in one launch: pre [T, B, 4H] = x.W for every step, without the bias [4H], which is added inside
 void lstm_recurrent_persistent(const Array& pre, const Array& bias, const Array& U, const Array& h0, const Array& c0, const Array& hs, const Array& c_out);
+// the same for a GRU: pre [T, B, 3H] = x.W + bias
 void gru_recurrent_persistent(const Array& pre, const Array& U, const Array& h0, const Array& hs, const Array& scratch);
 // softmax of a contiguous fp32 buffer seen as [outer, extent, inner] along `extent`, one pass over memory (records itself like any other launch)
 void softmax_axis_launch(const Array& x, const Array& out, long long outer, int extent, long long inner);
-// stride-1 convolution of a dense float NHWC image [N,H,W,C] (C a multiple of 4) with filters [O,fh,fw,C], fh <= 8:
-// one padding copy and one multi-term product, no patch matrix; returns [N, out_h, out_w, O]
+// convolution of a float NHWC image without padding, at any stride, with filters [f,fh,fw,C] (`other`), or the gradient of its filters (`other`: that of the
+// result), as one product that reads the image window by window. False, with nothing evaluated, where the library does not take the size; else
+// both operands have been evaluated and *result has `result_shape`
 bool conv2d_windows_nhwc(bool filters_gradient, const Array& image, const Array& other, const std::vector<int>& result_shape, int f, int fh, int fw, int stride_h, int stride_w,
                          Array* result);
+// stride-1 convolution of a dense float NHWC image [N,H,W,C] (C a multiple of 4) with filters [O,fh,fw,C], fh <= 8:
+// one padding copy and one multi-term product, no patch matrix; returns [N, out_h, out_w, O]
 Array conv2d_direct_nhwc(const Array& x, const Array& filters, int pad_top, int pad_left, int pad_bottom, int pad_right);
 // column numbers of the k best entries of every row of a [rows, cols] matrix, best first (evaluates its argument)
 Array topk_rows(const Array& x2d, int k, bool largest, bool ties_by_descending_column);

@@ -311,7 +311,8 @@ int dali_hip_lstm_step_small(int batch, int input, int hidden, const float* X, i
  */
 int dali_hip_lstm_recurrent_persistent(int steps, int batch, int hidden, const float* pre, const float* U, int ldu, const float* h0,
                                        const float* c0, float* hs, float* c_out);
-/* The same with the bias [4 hidden] apart: pre holds x(t).W alone and (pre + bias) stands in its place (bias may be NULL). */
+/* The same with the bias [4 hidden] apart: pre holds x(t).W alone and (pre + bias) stands in its place (bias may be NULL).
+ * hs must not overlap the bias either. */
 int dali_hip_lstm_recurrent_persistent_bias(int steps, int batch, int hidden, const float* pre, const float* bias, const float* U, int ldu, const float* h0,
                                             const float* c0, float* hs, float* c_out);
 /* Whether dali_hip_lstm_recurrent_persistent serves this batch and hidden size on the bound device: 0 no (the call would be refused), 1 yes,
