@@ -544,9 +544,9 @@ extern "C" int dali_hip_lstm_recurrent_persistent_supported(int batch, int hidde
     if (cus <= 0 || batch < 1) return 0;
     if (!lds_kernel_serves(batch, hidden, cus) && !recurrent_phased_supported(batch, hidden, cus)) return 0;
     // Measured against one fused launch per step, whose inner extent is cut into one share per compute unit at these batches
-    // (us per step over 32 steps, persistent / per step). 1024 hidden units: 6.2 / 16.7 at 8 rows, 11.7 / 17.2 at 32, 16.3 / 17.9 at
-    // 48, 18.8 / 18.3 at 64, 30.8 / 25.0 at 96; 512: 7.3 / 11.4 at 32, 11.7 / 11.7 at 48, 14.0 / 12.0 at 64; 2048: 27.3 / 40.2 at 32,
-    // 40.2 / 40.7 at 48, 52.8 / 40.7 at 64, 104 / 67 at 128.
+    // (us per step over 32 steps with the product of the input half, persistent / per step). 1024 hidden units: 5.4 / 16.0 at 8 rows, 10.6 / 16.3 at
+    // 32, 14.9 / 16.9 at 48, 16.5 / 17.2 at 64, 28.4 / 24.0 at 96; 512: 6.1 / 11.0 at 32, 9.9 / 11.4 at 48, 11.8 / 11.8 at 64; 2048: 24.1 / 39.3 at
+    // 32, 35.9 / 39.7 at 48, 47.3 / 40.1 at 64, 97 / 62 at 128; 768: 12.9 / 13.6 at 48. (The line was drawn where the persistent form was slower than it is now.)
     return batch <= 32 || (batch <= 48 && hidden >= 1024) ? 2 : 1;
 }
 
@@ -601,8 +601,8 @@ extern "C" int dali_hip_lstm_recurrent_persistent_bias(int steps, int batch, int
         if (e == hipSuccess) hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds_bytes, stream(), a);
     };
     const int KQ = hidden / 64;
-    // Waiting on the values themselves beats the barrier up to 32 rows (3.7 / 4.9 / 8.8 us a step at 1 / 8 / 32 rows of
-    // 1024 units against 6.6 / 7.5 / 10.3); from 33 rows on the tiles that have to be fetched a second time cost more than
+    // Waiting on the values themselves beats the barrier up to 32 rows (3.7 / 4.6 / 8.3 us a step at 1 / 8 / 32 rows of
+    // 1024 units against 8.3 / 9.3 / 10.5); from 33 rows on the tiles that have to be fetched a second time cost more than
     // the barrier (before the weights were in registers 12.8 against 11.3 us at 33 rows, 17.4 against 13.6 at 64). DALI_HIP_PERSISTENT_DATA_FLAGS=0: always barriers.
     static const bool flags_allowed = !(getenv("DALI_HIP_PERSISTENT_DATA_FLAGS") && atoi(getenv("DALI_HIP_PERSISTENT_DATA_FLAGS")) == 0);
     const bool data_flags = flags_allowed && MT <= 2;
